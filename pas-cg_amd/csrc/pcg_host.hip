@@ -375,6 +375,7 @@ struct DeviceBatch {
   Arena arena;
   int max_nlcap = 0, max_n = 0, max_items = 0;
   int max_nnc = 0;  // most native contacts of one system
+  bool lean = false;  // served job: the lean kernels carry it (once staged)
   int cell_words = 0;  // row-mask words of the largest system on a cell grid
   size_t bytes = 0;
   std::vector<Ran2> ran2;  // per system, RAN2 noise mode
@@ -1191,6 +1192,27 @@ int check_overflow(DeviceBatch &B) {
   return PCG_OK;
 }
 
+// Whether the lean kernels (LEAN in pcg_persist.hpp) carry everything this
+// batch can meet, once its bonded items are staged in LDS: chain-local bonded
+// items, complex native dihedrals, no disulfide potential on a contact, no
+// relative Debye-Hueckel term, no walls, and no PID pair. With QA on, the free
+// pairs take every pair PID would see but same-chain pairs four apart when QA
+// excludes those, so PID has pairs only if QA excludes them and PID does not.
+bool lean_batch(const DeviceBatch &B) {
+  const pcg_params &p = B.hp.p;
+  if (p.nat_dih_on && p.nat_dih_variant != 0) return false;
+  if (p.dh_on && p.dh_variant != 0) return false;
+  if (p.pid_on && !(p.qa_on && (p.qa_include4 || !p.pid_include4))) return false;
+  if (B.hp.solid_on || B.hp.hw_terms || B.hp.ljw_terms) return false;
+  for (const SysDesc &d : B.sys)
+    if (!d.bond_regular) return false;
+  if (p.nc_ss_kind != 0)
+    for (const HostSys &h : B.hs)
+      for (uint8_t t : h.nc_type)
+        if ((t & 0x7F) == 5) return false;
+  return true;
+}
+
 size_t lds_for(const DeviceBatch &B, bool staged) {
   return LdsLayout((size_t)B.max_n, sizeof(double), staged, false, (size_t)B.max_nnc).total;  // FP64 LDS forces
 }
@@ -1204,6 +1226,7 @@ struct PersistentCfg {
   bool ok;
   int block;
   size_t lds;
+  bool lean;  // the lean kernels
 };
 PersistentCfg persistent_cfg(DeviceBatch &B) {
   bool staged = lds_for(B, true) <= LDS_DYN_MAX;
@@ -1218,6 +1241,7 @@ PersistentCfg persistent_cfg(DeviceBatch &B) {
   int want = 64;
   while (want < 1024 && want < B.max_n * 2) want *= 2;
   c.block = std::min(std::max(want, 128), 512);
+  c.lean = staged && lean_batch(B);
   return c;
 }
 
@@ -1242,7 +1266,7 @@ struct pcg_ctx {
   int64_t steps_since_check = 0;
   int form = PCG_FORM_AUTO;  // requested
   int last_form = FORM_NONE;
-  PersistentCfg pcfg{false, 0, 0};
+  PersistentCfg pcfg{false, 0, 0, false};
   int spl = 500;             // persistent form: steps per launch
   ~pcg_ctx() {
     if (gexec) (void)hipGraphExecDestroy(gexec);
@@ -1386,7 +1410,7 @@ int pcg_step(pcg_ctx *c, int32_t nsteps) {
   if (use_persistent(*c)) {
     if ((rc = switch_form(*c, FORM_PERSISTENT))) return rc;
     for (int done = 0; done < nsteps; done += c->spl)
-      launch_persistent(B.d, B.prec, c->pcfg.block, std::min(c->spl, nsteps - done),
+      launch_persistent(B.d, c->pcfg.lean, B.prec, c->pcfg.block, std::min(c->spl, nsteps - done),
                         c->pcfg.lds, B.stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(B.stream));
@@ -1826,6 +1850,7 @@ struct pcg_batch {
   std::unique_ptr<DeviceBatch> B;
   int block = 0, spl = 0;  // threads per workgroup, steps per launch
   bool persistent = true;
+  bool lean = false;
   bool use_graph = false;
   size_t lds = 0;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -1862,7 +1887,7 @@ int run_persistent(pcg_batch *b, int nsteps) {
       b->gexec = nullptr;
       b->graph = nullptr;
       HIPCHK(hipStreamBeginCapture(B.stream, hipStreamCaptureModeThreadLocal));
-      launch_persistent(B.d, B.prec, b->block, b->spl, b->lds, B.stream);
+      launch_persistent(B.d, b->lean, B.prec, b->block, b->spl, b->lds, B.stream);
       HIPCHK(hipStreamEndCapture(B.stream, &b->graph));
       HIPCHK(hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
       b->g_block = b->block;
@@ -1870,11 +1895,11 @@ int run_persistent(pcg_batch *b, int nsteps) {
     }
     HIPCHK(hipEventRecord(b->ev0, B.stream));
     for (int k = 0; k < full; ++k) HIPCHK(hipGraphLaunch(b->gexec, B.stream));
-    if (rem) launch_persistent(B.d, B.prec, b->block, rem, b->lds, B.stream);
+    if (rem) launch_persistent(B.d, b->lean, B.prec, b->block, rem, b->lds, B.stream);
   } else {
     HIPCHK(hipEventRecord(b->ev0, B.stream));
     for (int done = 0; done < nsteps; done += b->spl)
-      launch_persistent(B.d, B.prec, b->block, std::min(b->spl, nsteps - done), b->lds, B.stream);
+      launch_persistent(B.d, b->lean, B.prec, b->block, std::min(b->spl, nsteps - done), b->lds, B.stream);
   }
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(b->ev1, B.stream));
@@ -1919,6 +1944,7 @@ int pcg_batch_create(const pcg_params *p, int32_t nsys, const pcg_model *models,
   const PersistentCfg pc = persistent_cfg(B);
   b->lds = pc.lds;
   b->persistent = pc.ok;
+  b->lean = pc.lean;
   if (opt.block != 0 && (opt.block < 64 || opt.block > 1024 || opt.block % 64 != 0))
     return fail(PCG_E_ARG, "block must be a multiple of 64 in [64, 1024]");
   if (opt.steps_per_launch < 0) return fail(PCG_E_ARG, "steps_per_launch must be >= 0");
@@ -2777,6 +2803,7 @@ int serve_launch(pcg_server *s, int k) {
     round = std::max<int64_t>(round, std::min<int64_t>(rem, 4 * (int64_t)s->o.chunk_steps));
   }
   size_t lds = 0;
+  bool lean = true;  // every job of the launch
   for (int q = 0; q < nres; ++q) {
     Job &j = *s->jobs[bk.resident[q]];
     DeviceBatch &B = *j.B;
@@ -2787,6 +2814,7 @@ int serve_launch(pcg_server *s, int k) {
     B.d.bond_lds = LdsLayout(nj, fsz, true, false, cj).total <= LDS_DYN_MAX ? 1 : 0;
     B.d.gear_lds = B.d.bond_lds && LdsLayout(nj, fsz, true, true, cj).total <= LDS_DYN_MAX ? 1 : 0;
     lds = std::max(lds, LdsLayout(nj, fsz, B.d.bond_lds != 0, B.d.gear_lds != 0, cj).total);
+    lean = lean && B.d.bond_lds && B.lean;
     bk.h_jobs[q] = B.d;
   }
   if (lds > LDS_DYN_MAX) return fail(PCG_E_ARG, "job too large for the persistent kernel");
@@ -2794,7 +2822,7 @@ int serve_launch(pcg_server *s, int k) {
                         bk.stream));
   HIPCHK(hipMemcpyAsync(bk.d_slots, bk.h_slots, nres * sizeof(JobSlot), hipMemcpyHostToDevice,
                         bk.stream));
-  launch_persistent_jobs(bk.d_jobs, bk.d_slots, nres, s->o.precision, SERVE_BUCKET_BLOCK[k],
+  launch_persistent_jobs(bk.d_jobs, bk.d_slots, nres, lean, s->o.precision, SERVE_BUCKET_BLOCK[k],
                          (int)round, lds, bk.stream);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(bk.h_slots, bk.d_slots, nres * sizeof(JobSlot), hipMemcpyDeviceToHost,
@@ -2869,6 +2897,7 @@ int serve_admit(pcg_server *s) {
       HIPCHK(hipMemcpyAsync((void *)j.B->d.sys, &d, sizeof(SysDesc), hipMemcpyHostToDevice,
                             bk.stream));
     }
+    j.B->lean = lean_batch(*j.B);
     j.status = PCG_JOB_RUNNING;
     j.t_start = now_s();
     j.block_bytes = blk_bytes;

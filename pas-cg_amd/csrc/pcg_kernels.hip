@@ -576,7 +576,7 @@ template <typename R, typename RF> __global__ void k_terms(DevBatch b, int only_
   AccG<RF> acc{(RF *)b.F[0], (RF *)b.F[1], (RF *)b.F[2]};
   double v = 0.0;
   for (int k = lo + blockIdx.x * blockDim.x + threadIdx.x; k < hi; k += gridDim.x * blockDim.x)
-    v += eval_item<R>(b, sd, st, g, acc, term, k);
+    v += eval_item<R>(b, sd, st, g, acc, term, k, st.t);
   v = block_sum(v);
   if (threadIdx.x == 0 && v != 0.0) atomicAdd(&st.V[term], v);
 }

@@ -155,19 +155,19 @@ __device__ __forceinline__ bool term_on(DevParamsC &P, int term) {
   return false;
 }
 
-// One item k (local to the system's list) of one term. Pair terms run in R;
+// One item k (local to the system's list) of one term, at time t. Pair terms run in R;
 // the angular terms, tethers, local repulsion, chirality, PID and the AFM
 // tips in FP64 (acos near 0/pi and the heuristic-angle polynomial lose too
 // much in FP32).
 template <typename R, typename G, typename A>
 __device__ __forceinline__ double eval_item(const DevBatch &b, SysDescC &s, SysState &st,
-                                            const G &g, A &acc, int term, int k,
+                                            const G &g, A &acc, int term, int k, double t,
                                             bool want_v = true) {
   switch (term) {
   case PCG_CHIR: return chir_item<double>(b, g, acc, s.chir0 + k);
   case PCG_TETHER: return tether_item<double>(b, g, acc, s.teth0 + k);
   case PCG_LREP: return lrep_item<double>(b, g, acc, s.lrep0 + k);
-  case PCG_NAT_CONT: return nat_cont_item<R>(b, s, st, g, acc, s.nc0 + k, st.t);
+  case PCG_NAT_CONT: return nat_cont_item<R>(b, s, st, g, acc, s.nc0 + k, t);
   case PCG_PAULI: return pauli_item<R>(b, s, g, acc, s.nl0 + k);
   case PCG_CONST_DH: return dh_item<R>(b, s, g, acc, s.nl0 + k, 0, want_v);
   case PCG_REL_DH: return dh_item<R>(b, s, g, acc, s.nl0 + k, 1, want_v);
@@ -179,8 +179,8 @@ __device__ __forceinline__ double eval_item(const DevBatch &b, SysDescC &s, SysS
   case PCG_HEUR_DIH: return heur_dih_item<double>(b, g, acc, s.hdih0 + k);
   case PCG_CND: return nat_dih_item<double>(b, g, acc, s.ndih0 + k, 0);
   case PCG_SND: return nat_dih_item<double>(b, g, acc, s.ndih0 + k, 1);
-  case PCG_VEL_AFM: return vel_afm_item<double>(b, g, acc, s.tip0 + k, st.t - s.afm_t0, st.t);
-  case PCG_FORCE_AFM: return force_afm_item(b, acc, s.tip0 + s.ntip + k, st.t);
+  case PCG_VEL_AFM: return vel_afm_item<double>(b, g, acc, s.tip0 + k, t - s.afm_t0, t);
+  case PCG_FORCE_AFM: return force_afm_item(b, acc, s.tip0 + s.ntip + k, t);
   case PCG_SOLID_WALL: return solid_wall_item(b, g, acc, s.res0 + k);
   case PCG_HW_FREE: return hw_free_item(b, g, acc, s.res0 + k);
   case PCG_HW_CONN: return hw_conn_item(b, g, acc, k);

@@ -26,11 +26,16 @@ void launch_ljw_process(const DevBatch &b, hipStream_t s);
 void launch_box_setup(const DevBatch &b, DevParams *P, SysDesc *sd, hipStream_t s);
 void launch_box_phase(const DevBatch &b, DevParams *P, SysDesc *sd, hipStream_t s);
 void launch_box_log(const DevBatch &b, hipStream_t s);
-// persistent form: every system of the batch advances nsteps in one launch
-void launch_persistent(const DevBatch &b, int prec, int block, int nsteps, size_t lds_bytes,
+// persistent form: every system of the batch advances nsteps in one launch;
+// lean: the lean kernels (pcg_batch_lean.hip), for batches lean_batch allows
+void launch_persistent(const DevBatch &b, bool lean, int prec, int block, int nsteps,
+                       size_t lds_bytes, hipStream_t s);
+void launch_persistent_jobs(const DevBatch *jobs, JobSlot *slots, int njobs, bool lean, int prec,
+                            int block, int nsteps, size_t lds_bytes, hipStream_t s);
+void launch_batch_lean(const DevBatch &b, int prec, int block, int nsteps, size_t lds_bytes,
                        hipStream_t s);
-void launch_persistent_jobs(const DevBatch *jobs, JobSlot *slots, int njobs, int prec, int block,
-                            int nsteps, size_t lds_bytes, hipStream_t s);
+void launch_jobs_lean(const DevBatch *jobs, JobSlot *slots, int njobs, int prec, int block,
+                      int nsteps, size_t lds_bytes, hipStream_t s);
 // report sums of every system (pcg_report.hip)
 void launch_report(const DevBatch &b, int pid_on, ReportSums *out, hipStream_t s);
 // the same into the library's own device array (no allocation), for batches

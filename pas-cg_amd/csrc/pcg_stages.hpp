@@ -265,9 +265,9 @@ __device__ inline void qa_finish_block(const DevBatch &b, SysDescC &sd, SysState
 // (cg/include/cg/langevin/step.h:10-12). The displacement from the last NL
 // rebuild is reduced here for the next step's verify.
 // ya(k, c) is a reference to y_k, component c, of the residue (in HBM or LDS)
-// minv = 1 / mass and sqminv = sqrt(minv) of the residue's type.
+// minv = 1 / mass and sqminv = sqrt(minv) of the residue's type; t0: time 0.
 template <typename YA>
-__device__ __forceinline__ void gear_core(const DevBatch &b, SysDescC &sd, const SysState &st,
+__device__ __forceinline__ void gear_core(const DevBatch &b, SysDescC &sd, bool t0,
                                           double minv, double sqminv, double Fx, double Fy,
                                           double Fz, const double nz[3], double out_r[3],
                                           double vel[3], YA ya) {
@@ -281,7 +281,7 @@ __device__ __forceinline__ void gear_core(const DevBatch &b, SysDescC &sd, const
   for (int c = 0; c < 3; ++c) {
     double y0 = ya(0, c), y1 = ya(1, c), y2 = ya(2, c), y3 = ya(3, c), y4 = ya(4, c),
            y5 = ya(5, c);
-    if (st.t == 0) y2 = F[c] * P.deltsq;
+    if (t0) y2 = F[c] * P.deltsq;
     double f = F[c] - gam2 * y1;
     y1 = y1 + con2 * nz[c];
     double err = y2 - P.deltsq * f;
@@ -312,7 +312,7 @@ __device__ __forceinline__ void gear_update(const DevBatch &b, SysDescC &sd, con
                                             const double nz[3], double out_r[3]) {
   double vel[3];
   const double minv = 1.0 / b.P->p.mass[b.atype[i]];
-  gear_core(b, sd, st, minv, sqrt(minv), Fx, Fy, Fz, nz, out_r, vel,
+  gear_core(b, sd, st.t == 0, minv, sqrt(minv), Fx, Fy, Fz, nz, out_r, vel,
             [&](int k, int c) -> double & { return b.y[k][c][i]; });
   for (int c = 0; c < 3; ++c) b.vel[c][i] = vel[c];
 }
