@@ -115,51 +115,80 @@ __device__ __forceinline__ double block_max(double v, double *part) {
 // Tallies of the list rebuild: NL pairs, then the pairs of each list the
 // ordered partition fills (native contacts, QA free pairs, the QA free pairs
 // that can become candidates, PID, DH, Pauli).
+enum { KC_NEAR = 1, KC_PID = 2, KC_DH = 4, KC_PAULI = 8 };  // a kept pair's lists
 enum { RB_NL = 0, RB_NC, RB_QA, RB_NEAR, RB_PID, RB_DH, RB_PAULI, RB_N };
 
-// First row of wave w's block when nw waves split rows 0..n-1 of the
-// upper-triangle pair rows (row k holds n - 1 - k pairs) into contiguous
-// blocks of about equal pair counts: the smallest k with
-// k (n - 1) - k (k - 1) / 2 >= w P / nw, P = n (n - 1) / 2. Monotone in w,
-// 0 for w = 0 and n for w = nw.
+// Cost of the rows before row k in the rebuild's first pass, in 64-column
+// chunks: row k visits the chunks from its next residue's to the last, and
+// costs about a chunk and a half of its own.
+__device__ __forceinline__ int rb_cost(int k, int n) {
+  const int W = (n + 63) >> 6, q = k >> 6, r = k & 63;
+  return 2 * (k * W - (32 * q * (q - 1) + q * (r + 1))) + 3 * k;  // in half chunks
+}
+// First row of wave w's block when nw waves split the rows into contiguous
+// blocks of about equal cost. Monotone in w, 0 for w = 0 and n for w = nw.
 __device__ __forceinline__ int rb_row_start(int w, int nw, int n) {
   if (w <= 0) return 0;
   if (w >= nw) return n;
-  const double P = 0.5 * (double)n * (double)(n - 1);
-  const double T = P * (double)w / (double)nw;
-  const double h = (double)n - 0.5;
-  const double disc = fmax(h * h - 2.0 * T, 0.0);
-  int k = (int)ceil(h - sqrt(disc));
-  k = max(0, min(n, k));
-  // exact integer correction of the rounding
-  auto C = [&](long long kk) { return kk * (long long)(n - 1) - kk * (kk - 1) / 2; };
-  const long long Ti = (long long)ceil(T);
-  while (k > 0 && C(k - 1) >= Ti) --k;
-  while (k < n && C(k) < Ti) ++k;
-  return k;
+  const int want = (int)((float)rb_cost(n, n) * ((float)w / (float)nw));
+  int lo = 0, hi = n;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (rb_cost(mid, n) < want) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo;
+}
+
+__device__ __forceinline__ float lane_f32(float v, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+
+__device__ __forceinline__ unsigned long long lane_u64(unsigned long long v, int lane) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane);
+  return (unsigned long long)lo | ((unsigned long long)hi << 32);
 }
 
 // nl::legacy_update (cg/src/cg/nl/legacy_update.cpp:11-55) fused with the
 // ordered list updates of thread_main.cpp:409-423 and the QA near list,
 // inside the workgroup and without writing the NL itself. The rows of the
 // sorted NL (pairs i < j) are split into contiguous blocks of about equal
-// pair counts, one per wave; a wave walks its rows in order, 64 columns j at
-// a time, and classifies every pair on the spot as the partition would
-// classify the NL pair: native contact (a taken pair of the row's native
-// contacts), QA free pair (taken), PID bundle, DH pair, Pauli pair. A first
-// pass counts each list's pairs per wave, a scan over the waves gives each
-// wave its offsets, and a second pass writes every pair at its wave's
-// offset plus its rank among the block's earlier pairs of that list (a
-// running count and a ballot): the lists come out exactly in the order of
-// partitioning the sorted NL. The counts are scalars; nothing per row goes
-// to memory.
+// cost, one per wave, and handled in three stages:
 //
-// Every decision is the FP64 one of the reference's expressions. The squared
-// distance is formed in FP32 from the FP64 differences; when it is clear of
-// every threshold by a relative 2e-5 (far beyond FP32's rounding of a sum of
-// three squares) the FP32 comparison decides, else the exact FP64 distance
-// does. The FP64 distance itself is formed for the pairs whose lists keep it
-// (QA near pairs, PID bundles).
+// scan      each row against every later column, 64 at a time: the pairs
+//           within the NL radius and within the native-contact radius are
+//           counted, the pairs that may join a list kept in order;
+// classify  the kept pairs, 64 at a time, as the partition would classify the
+//           NL pair (native contacts and QA free pairs take; PID bundle, DH
+//           pair, Pauli pair), by their exact FP64 distance;
+// write     once a scan over the waves has given each wave its offsets: every
+//           kept pair at its wave's offset plus its rank among the block's
+//           earlier pairs of that list, so the lists come out exactly in the
+//           order of partitioning the sorted NL.
+//
+// The native contacts come from their own sorted list, which is the NL's
+// order, a contiguous run of contacts a wave.
+//
+// The scan tests all n (n - 1) / 2 pairs. It is bound by the instructions each
+// wave runs through one after another (measured: 5 cycles a dependent vector
+// instruction, 7 a scalar one, 10 where a scalar one waits for a compare),
+// not by the vector unit: classifying each 64 columns on the spot took 2500
+// cycles for them, mostly scalar logic and branches. Now 64 columns cost one
+// 16-byte LDS read of FP32 positions (relative to residue 0, staged over the
+// force accumulators, which are zero during a rebuild), the squared distance,
+// two counts and one test for every reason to keep a pair; the row's data come
+// from registers by readlane. A rebuild of a 600-residue protein on 1024
+// threads takes 95 us instead of 280, of a 56-residue one 15 us instead of 41.
+//
+// Every decision is the FP64 one of the reference's expressions. The scan's
+// FP32 comparison counts a pair when its squared distance is clear of the
+// threshold by a relative margin of 2e-5 + 1e-6 M / d (M the largest
+// coordinate staged, d the threshold): staging rounds a coordinate by at most
+// 2^-24 M and the difference, squares and sums round by at most a few 2^-24,
+// together less than 4.2e-7 M / d + 4e-7. Pairs inside a margin are kept and
+// counted by the classification. In a periodic cell the differences are
+// formed and wrapped in FP64 and rounded afterwards (M = 0).
 //
 // QA free pairs beyond the QA maximum required distance are counted (qf_n,
 // which sizes the contact loop as the reference's free-pair count does) but
@@ -169,13 +198,16 @@ __device__ __forceinline__ int rb_row_start(int w, int nw, int n) {
 // their relative order, so the (distance, free-pair index) order of the QA
 // finish is unchanged.
 //
-// The chain and sequence indices of the residues, the row starts of the
-// static native contacts and the contacts' second residues sit in the LDS
-// region of the QA stacks (rb), which is free during a rebuild.
+// rb: the LDS region of the QA stacks, free during a rebuild: the residues'
+// sequence words, the row starts of the static native contacts and the
+// contacts' second residues. force: the force accumulators (24 n bytes from a
+// multiple of 8, zero again after); pos4: the multiple of 16 from there.
 // (inlined: as a call it would make the kernel save every live register)
 __device__ __forceinline__ void wg_fix_nl(DevBatchC *bp, int s, SysState &st, const GeoL &g,
-                                          void *rb) {
+                                          void *rb, double *force, float4 *pos4,
+                                          uint32_t chg) {
 #pragma clang fp contract(off)
+  typedef unsigned long long u64;
   const DevBatch b = unpack(bp);
   SysDescC &sd = b.sys[s];
   DevParamsC &P = *b.P;
@@ -185,7 +217,6 @@ __device__ __forceinline__ void wg_fix_nl(DevBatchC *bp, int s, SysState &st, co
   // are then scalar loops and the running counts scalar registers
   const int nw = blockDim.x >> 6, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const unsigned long long below = (1ull << lane) - 1ull;
   const int nnc = p.nat_cont_on ? sd.nnc : 0;
   // each residue's sequence index, chain and type in one word (seq | chain
   // << 12 | type << 24: a persistent system has fewer than 4096 residues)
@@ -193,10 +224,40 @@ __device__ __forceinline__ void wg_fix_nl(DevBatchC *bp, int s, SysState &st, co
   int *rs = (int *)(csq + n);  // rs[0..n]
   uint16_t *pj = (uint16_t *)(rs + n + 1);               // [nnc]
   __shared__ int wcnt[16][RB_N];
+  __shared__ float wspan[16];
+  __shared__ int wirr[16];
+  __shared__ u64 charge_mask[64];  // the charged residues of each 64
   const bool cell = has_cell(sd);
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    csq[k] = (uint32_t)b.seq[r0 + k] | ((uint32_t)b.chain[r0 + k] << 12) |
-             ((uint32_t)(g.at[k] & 63) << 24);
+  const double ox = g.x[0], oy = g.y[0], oz = g.z[0];
+  float span = 0.0f;
+  bool irr = false;
+  for (int k0 = threadIdx.x - lane; k0 < n; k0 += blockDim.x) {
+    const int k = k0 + lane;
+    const u64 cm = __ballot(k < n && ((chg >> (g.at[min(k, n - 1)] & 31)) & 1u));
+    if (lane == 0) charge_mask[k0 >> 6] = cm;
+    if (k >= n) continue;
+    const int ch = b.chain[r0 + k], sq = b.seq[r0 + k];
+    csq[k] = (uint32_t)sq | ((uint32_t)ch << 12) | ((uint32_t)(g.at[k] & 63) << 24);
+    // the usual numbering: chains one after another, consecutive sequence
+    // indices within one; then a pair's sequence distance is j - k, and the
+    // exclusions concern only the four columns after the row's residue: bit
+    // d - 1 of mate tells whether residue k + d is of the same chain
+    uint32_t mate = 0u;
+    for (int d = 1; d <= 4; ++d)
+      if (k + d < n && b.chain[r0 + k + d] == ch) mate |= 1u << (d - 1);
+    if (k + 1 < n) {
+      const int c1 = b.chain[r0 + k + 1];
+      irr |= c1 < ch || (c1 == ch && b.seq[r0 + k + 1] != sq + 1);
+    }
+    const float fx = (float)(g.x[k] - ox), fy = (float)(g.y[k] - oy), fz = (float)(g.z[k] - oz);
+    span = fmaxf(span, fmaxf(fabsf(fx), fmaxf(fabsf(fy), fabsf(fz))));
+    pos4[k] = make_float4(fx, fy, fz, __builtin_bit_cast(float, (uint32_t)(g.at[k] & 31) | (mate << 8)));
+  }
+  for (int o = 32; o > 0; o >>= 1) span = fmaxf(span, __shfl_down(span, o, 64));
+  const bool wave_irr = __any(irr);
+  if (lane == 0) {
+    wspan[w] = span;
+    wirr[w] = wave_irr;
   }
   // contacts sd.nc0 + [rs[k], rs[k + 1]) of the list sorted by (i1, i2) are
   // those of residue r0 + k with later residues; pj holds their second
@@ -220,215 +281,344 @@ __device__ __forceinline__ void wg_fix_nl(DevBatchC *bp, int s, SysState &st, co
   const double t_rep = __dadd_rn(p.rep_cutoff, pad);
   const double t_near = P.qa_max_req;
   const double rt_dh = __ddiv_rn(1.0, t_dh);
-  // squared thresholds in FP32, and their margins
-  const float s_nl = (float)(t_nl * t_nl), s_nc = (float)(t_nc * t_nc), s_dh = (float)(t_dh * t_dh),
-              s_rep = (float)(t_rep * t_rep), s_near = (float)(t_near * t_near);
-  const float mlo = 1.0f - 2e-5f, mhi = 1.0f + 2e-5f;
-  const float e_nl[2] = {s_nl * mlo, s_nl * mhi}, e_nc[2] = {s_nc * mlo, s_nc * mhi},
-              e_dh[2] = {s_dh * mlo, s_dh * mhi}, e_rep[2] = {s_rep * mlo, s_rep * mhi},
-              e_near[2] = {s_near * mlo, s_near * mhi};
-  const float e_far = fmaxf(fmaxf(fmaxf(e_nl[1], e_nc[1]), fmaxf(e_dh[1], e_rep[1])), e_near[1]);
   const bool qa_on = p.qa_on, pid_on = p.pid_on, dh_on = p.dh_on, pauli_on = P.pauli_on;
   const bool qa4 = p.qa_include4, pid4 = p.pid_include4;
-  // residue types with a charge, as bits (q1 q2 != 0 iff both are set)
-  uint32_t chg = 0u;
-  for (int t = 0; t < 21; ++t) chg |= (p.charge[t] != 0.0 ? 1u : 0u) << t;
-  const int kbeg = rb_row_start(w, nw, n), kend = rb_row_start(w + 1, nw, n);
-  // When every pair fits the NL capacity, the first pass also stores, in
-  // order, the wave's pairs that the second pass writes somewhere (native
-  // contacts, QA near pairs, PID, DH and Pauli pairs; QA free pairs beyond
-  // the near distance are only counted): k | j << 16 in nl_i[0], the
-  // classes in nl_cls, a native contact's index in nl_i[1], from the index
-  // of its block's first pair, which no other wave's pairs reach. The
-  // second pass walks those instead of every pair of the block.
-  const bool compact = (long long)n * (n - 1) / 2 <= (long long)sd.nlcap;
-  const int seg = sd.nl0 + (int)((long long)kbeg * (n - 1) - (long long)kbeg * (kbeg - 1) / 2);
-  int my_nl = 0;
-  // the second pass's writes of one pair: native contact c, QA free pair
-  // and near-list entry, PID bundle, DH pair, Pauli pair, each at the wave's
-  // running offset plus its rank among the chunk's earlier pairs of the list
-  auto emit = [&](int k, int j, int c, bool is_nc, bool near, bool is_pid, bool is_dh,
-                  bool is_pauli, unsigned long long m_nc, unsigned long long m_near,
-                  unsigned long long m_pid, unsigned long long m_dh, unsigned long long m_pauli,
-                  const int *off) {
-    const int i = r0 + k, jg = r0 + j;
-    const int ai = g.at[k] & 63, aj = g.at[j] & 63;
-    if (is_nc) b.ncur[sd.nc0 + off[RB_NC] + __popcll(m_nc & below)] = c;
-    double d64 = 0.0;
-    if (near | is_pid) {
-      v3<double> dd = xsub(v3<double>{g.x[j], g.y[j], g.z[j]}, v3<double>{g.x[k], g.y[k], g.z[k]});
-      if (cell) dd = xwrapd(dd, sd);
-      d64 = xnorm3(dd);
-    }
-    if (near) {
-      const int f = off[RB_NEAR] + __popcll(m_near & below);
-      if (f < sd.qfcap) {
-        const int q = sd.qf0 + f;
-        b.qf_i[0][q] = i;
-        b.qf_i[1][q] = jg;
-        b.qf_d[q] = d64;
-        b.qf_vac[q] = 0;
-        // near list entry f: the free pair in slot f
-        const double req = fmax(fmax(fmax(g.req_t[1], g.req_t[2]), g.req_t[3]),
-                                g.req_t[4 + ai + 21 * aj]);
-        const double thr = fmin(P.qa_max_req, fmax(p.rep_cutoff, req)) * (1.0 + 1e-5);
-        b.qh_slot[q] = f;
-        b.qh_i[0][q] = i;
-        b.qh_i[1][q] = jg;
-        b.qh_vac[q] = 0;
-        b.qh_req[q] = req;
-        b.qh_thr2[q] = (float)(thr * thr);
-        b.qh_ij[q] = (uint32_t)k | ((uint32_t)j << 16);
-      }
-    }
-    if (is_pid) {
-      const int pos = off[RB_PID] + __popcll(m_pid & below);
-      if (pos < sd.nlcap) {
-        const int q = sd.nl0 + pos;
-        b.pid_i[0][q] = i;
-        b.pid_i[1][q] = jg;
-        b.pid_d[q] = d64;
-        b.pid_t[q] = (int16_t)(ai * 21 + aj);
-      }
-    }
-    if (is_dh) {
-      const int pos = off[RB_DH] + __popcll(m_dh & below);
-      if (pos < sd.nlcap) {
-        const int q = sd.nl0 + pos;
-        b.dh_i[0][q] = i;
-        b.dh_i[1][q] = jg;
-        b.dh_q[q] = p.charge[ai] * p.charge[aj];
-      }
-    }
-    if (is_pauli) {
-      const int pos = off[RB_PAULI] + __popcll(m_pauli & below);
-      if (pos < sd.nlcap) {
-        const int q = sd.nl0 + pos;
-        b.pauli_i[0][q] = i;
-        b.pauli_i[1][q] = jg;
-      }
-    }
-  };
   __syncthreads();
+  bool regular = true;
+  span = 0.0f;
+  for (int v = 0; v < nw; ++v) {
+    span = fmaxf(span, wspan[v]);
+    regular = regular && !wirr[v];
+  }
+  if (cell) span = 0.0f;
+  // squared thresholds in FP32, their margins (half) in the FP32 comparisons,
+  // and the bounds clear of them; in scalar registers
+  auto half = [&](double t) {
+    const float tf = (float)t;
+    return tf * tf * (2e-5f + 1e-6f * span * rcpR(tf));
+  };
+  auto sq32 = [&](double t) { return (float)(t * t); };
+  auto uni = [&](float x) { return lane_f32(x, 0); };
+  const float nl_c = uni(sq32(t_nl)), nc_c = uni(sq32(t_nc));
+  // the NL and native-contact radii share the wider of their margins
+  const float h_nl = uni(fmaxf(half(t_nl), half(t_nc)));
+  const float nl_lo = nl_c - h_nl, nl_hi = nl_c + h_nl, nc_lo = nc_c - h_nl, nc_hi = nc_c + h_nl;
+  const float band = h_nl * 1.001f;  // (with the comparison's own rounding)
+  const float dh_lo = uni(sq32(t_dh) - half(t_dh)), dh_hi = uni(sq32(t_dh) + half(t_dh));
+  const float near_lo = uni(sq32(t_near) - half(t_near)), near_hi = uni(sq32(t_near) + half(t_near));
+  const float rep_lo = uni(sq32(t_rep) - half(t_rep)), rep_hi = uni(sq32(t_rep) + half(t_rep));
+  // every pair this close is kept for the classification
+  float keep_to = -1.0f;
+  if (qa_on) keep_to = fmaxf(keep_to, near_hi);
+  if (pauli_on) keep_to = fmaxf(keep_to, rep_hi);
+  if (pid_on && !qa_on) keep_to = fmaxf(keep_to, nc_hi);
+  const float keep_c = keep_to * 1.00001f - band;
+  // pairs four apart are told apart by the lists' own options
+  const bool keep4 = (qa_on && !qa4) || (pid_on && !pid4);
+  const int kbeg = rb_row_start(w, nw, n), kend = rb_row_start(w + 1, nw, n);
+  // the kept pairs, k | j << 12 | classes << 24, go to nl_i[0]: when every
+  // pair fits the NL capacity a wave's region starts at the index of its
+  // block's first pair, which no other wave's pairs reach; else each wave has
+  // an equal share and takes its rows in batches whose pairs fit it, scanned
+  // and classified in both passes
+  const bool compact = (long long)n * (n - 1) / 2 <= (long long)sd.nlcap;
+  const int share = compact ? 0 : sd.nlcap / nw;
+  uint32_t *kp = (uint32_t *)b.nl_i[0] + sd.nl0 +
+                 (compact ? (int)((long long)kbeg * (n - 1) - (long long)kbeg * (kbeg - 1) / 2)
+                          : w * share);
+  const int batch = compact ? max(kend - kbeg, 1) : max(share / n, 1);
+  const int W = (n + 63) >> 6;
+  const u64 last_cols = (n & 63) ? ~0ull >> (64 - (n & 63)) : ~0ull;
+  const u64 charged = lane < W ? charge_mask[lane] : 0ull;  // of chunk l, in lane l
+  // the wave's native contacts: whole 64s of the list
+  const int nc64 = (nnc + 63) >> 6, cper = ((nc64 + nw - 1) / nw) << 6;
+  const int cbeg = min(w * cper, nnc), cend = min(cbeg + cper, nnc);
+  auto word_same = [&](uint32_t wa, uint32_t wb) {
+    return ((wa >> 12) & 0xFFFu) == ((wb >> 12) & 0xFFFu);
+  };
+  auto word_gap = [&](uint32_t wa, uint32_t wb) {
+    return abs((int)(wa & 0xFFFu) - (int)(wb & 0xFFFu));
+  };
+  auto pair_dist = [&](int k, int j) {
+    v3<double> dd = xsub(v3<double>{g.x[j], g.y[j], g.z[j]}, v3<double>{g.x[k], g.y[k], g.z[k]});
+    if (cell) dd = xwrapd(dd, sd);
+    return xnorm3(dd);
+  };
+  // a pair's squared distance as the scan sees it
+  auto scan_d2 = [&](float4 q, float xi, float yi, float zi, int k, int j) {
+    float dx = q.x - xi, dy = q.y - yi, dz = q.z - zi;
+    if (cell) {
+      const v3<double> dd = xwrapd(xsub(v3<double>{g.x[j], g.y[j], g.z[j]},
+                                        v3<double>{g.x[k], g.y[k], g.z[k]}), sd);
+      dx = (float)dd.x, dy = (float)dd.y, dz = (float)dd.z;
+    }
+    return __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+  };
+  auto rank_in = [&](u64 m, int base = 0) {  // base plus the earlier lanes of the mask
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, base));
+  };
+  const bool plain = regular && !cell && !keep4;
+  int kept = 0;
+  u64 native_in = 0ull;
   for (int pass = 0; pass < 2; ++pass) {
     int off[RB_N];
-    for (int c = 0; c < RB_N; ++c) off[c] = pass ? wcnt[w][c] : 0;
-    if (pass && compact) {
-      // the wave's NL pairs, 64 at a time, in the first pass's order
-      for (int t0 = 0; t0 < my_nl; t0 += 64) {
-        const int t = t0 + lane;
-        const bool v = t < my_nl;
-        const uint32_t kw = v ? (uint32_t)b.nl_i[0][seg + t] : 0u;
-        const int cls = v ? (int)b.nl_cls[seg + t] : 0;
-        const int k = (int)(kw & 0xffffu), j = (int)(kw >> 16);
-        const bool is_nc = cls & CL_NC, near = cls & CL_NEAR, is_pid = cls & CL_PID,
-                   is_dh = cls & CL_DH, is_pauli = cls & CL_PAULI;
-        const int c = is_nc ? b.nl_i[1][seg + t] : 0;
-        const unsigned long long m_nc = __ballot(is_nc), m_near = __ballot(near),
-                                 m_pid = __ballot(is_pid), m_dh = __ballot(is_dh),
-                                 m_pauli = __ballot(is_pauli);
-        if (v) emit(k, j, c, is_nc, near, is_pid, is_dh, is_pauli, m_nc, m_near, m_pid, m_dh,
-                    m_pauli, off);
-        off[RB_NC] += __popcll(m_nc);
-        off[RB_NEAR] += __popcll(m_near);
-        off[RB_PID] += __popcll(m_pid);
-        off[RB_DH] += __popcll(m_dh);
-        off[RB_PAULI] += __popcll(m_pauli);
+    for (int c = 0; c < RB_N; ++c) off[c] = pass ? __builtin_amdgcn_readfirstlane(wcnt[w][c]) : 0;
+    for (int ka = kbeg; ka < kend; ka += batch) {
+      const int kb = min(ka + batch, kend);
+      if (!pass || !compact) {
+        // ---- scan: the rows' pairs counted against the NL radius and the
+        // native-contact radius, the close ones and those in a margin kept
+        int lane_in = 0, lane_inner = 0;
+        kept = 0;
+        for (int kg = ka; kg < kb; kg += 64) {
+          const float4 rp = pos4[min(kg + lane, n - 1)];  // 64 rows' data, one a lane
+          const int kn = min(kb - kg, 64);
+          if (plain) {
+            // the next chunk's columns (or the next row's first) are loaded a
+            // chunk ahead
+            float4 nq = pos4[min((((kg + 1) >> 6) << 6) + lane, n - 1)];
+            for (int r = 0; r < kn; ++r) {
+              const int k = kg + r;
+              const float xi = lane_f32(rp.x, r), yi = lane_f32(rp.y, r), zi = lane_f32(rp.z, r);
+              const uint32_t wk = (uint32_t)__builtin_amdgcn_readlane(__builtin_bit_cast(int, rp.w), r);
+              const bool row_dh = dh_on && ((chg >> (wk & 31)) & 1u);
+              // the columns past the row's residue, without the two after it
+              // that are of its chain, in the row's first two chunks
+              const int sh = (k + 1) & 63;
+              const u64 ex = (wk >> 8) & 3u;
+              u64 cols = (~0ull << sh) & ~(ex << sh), cols1 = sh ? ~(ex >> (64 - sh)) : ~0ull;
+              for (int jc = (k + 1) >> 6; jc < W; ++jc) {
+                const int j = jc * 64 + lane;
+                const float4 q = nq;
+                nq = pos4[min(jc + 1 < W ? j + 64 : (((k + 2) >> 6) << 6) + lane, n - 1)];
+                if (jc == W - 1) cols &= last_cols;
+                const float dx = q.x - xi, dy = q.y - yi, dz = q.z - zi;
+                float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+                d2 = __builtin_amdgcn_inverse_ballot_w64(cols) ? d2 : 1e30f;
+                lane_in += d2 < nl_lo ? 1 : 0;
+                lane_inner += d2 < nc_lo ? 1 : 0;
+                // one test for all reasons to keep a pair: inside keep_to, or
+                // within band of the NL or the native-contact radius
+                const float why = fminf(fminf(fabsf(d2 - nl_c), fabsf(d2 - nc_c)), d2 - keep_c);
+                u64 keep = __ballot(why <= band);
+                if (row_dh) {
+                  u64 dm = lane_u64(charged, jc) & __ballot(d2 <= dh_hi);
+                  if (qa_on) dm &= ~__ballot(d2 < nc_lo);
+                  keep |= dm;
+                }
+                if (__builtin_amdgcn_inverse_ballot_w64(keep))
+                  *(uint32_t *)((char *)kp + 4u * (uint32_t)rank_in(keep, kept)) =
+                      (uint32_t)k | ((uint32_t)j << 12);
+                kept += __popcll(keep);
+                cols = cols1;
+                cols1 = ~0ull;
+              }
+            }
+          } else {
+            for (int r = 0; r < kn; ++r) {
+              const int k = kg + r;
+              const float xi = lane_f32(rp.x, r), yi = lane_f32(rp.y, r), zi = lane_f32(rp.z, r);
+              const uint32_t wi = csq[k];
+              const bool row_dh = dh_on && ((chg >> ((wi >> 24) & 31)) & 1u);
+              for (int jc = (k + 1) >> 6; jc < W; ++jc) {
+                const int j = jc * 64 + lane, jj = min(j, n - 1);
+                const float d2 = scan_d2(pos4[jj], xi, yi, zi, k, jj);
+                const uint32_t wj = csq[jj];
+                const bool same = word_same(wi, wj);
+                const u64 cols = __ballot(j > k & j < n & !(same & (word_gap(wi, wj) < 3)));
+                const bool col = __builtin_amdgcn_inverse_ballot_w64(cols);
+                lane_in += (col & (d2 < nl_lo)) ? 1 : 0;
+                lane_inner += (col & (d2 < nc_lo)) ? 1 : 0;
+                const float why = fminf(fminf(fabsf(d2 - nl_c), fabsf(d2 - nc_c)), d2 - keep_c);
+                u64 keep = __ballot(why <= band);
+                if (keep4) keep |= __ballot(same & (word_gap(wi, wj) == 4));
+                if (row_dh) {
+                  u64 dm = lane_u64(charged, jc) & __ballot(d2 <= dh_hi);
+                  if (qa_on) dm &= ~__ballot(d2 < nc_lo);
+                  keep |= dm;
+                }
+                keep &= cols;
+                if (__builtin_amdgcn_inverse_ballot_w64(keep))
+                  kp[rank_in(keep, kept)] = (uint32_t)k | ((uint32_t)j << 12);
+                kept += __popcll(keep);
+              }
+            }
+          }
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+          lane_in += __shfl_xor(lane_in, o, 64);
+          lane_inner += __shfl_xor(lane_inner, o, 64);
+        }
+        int n_in = __builtin_amdgcn_readfirstlane(lane_in);
+        int n_inner = __builtin_amdgcn_readfirstlane(lane_inner);
+        // the stores above before the loads of other lanes' pairs below
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        // ---- classify
+        int n_four = 0;
+        int cnt[RB_N] = {0};
+        uint32_t next = lane < kept ? kp[lane] : 0u;
+        for (int t0 = 0; t0 < kept; t0 += 64) {
+          const int t = t0 + lane;
+          const bool valid = t < kept;
+          const uint32_t word = next;
+          next = t + 64 < kept ? kp[t + 64] : 0u;
+          const int k = (int)(word & 0xFFFu), j = (int)((word >> 12) & 0xFFFu);
+          const float4 pk = pos4[k], pl = pos4[j];
+          // a native partner? the row's contacts, eight at a time
+          bool native = false;
+#pragma clang loop unroll(disable)
+          for (int c = rs[k], ce = rs[k + 1]; c < ce; c += 8) {
+            uint16_t e[8];
+            __builtin_memcpy(e, pj + c, 16);
+            for (int m = 0; m < 8; ++m) native |= (c + m < ce) & (e[m] == j);
+          }
+          const float d2 = scan_d2(pl, pk.x, pk.y, pk.z, k, j);
+          bool in = d2 < nl_lo, inner = d2 < nc_lo, b_near = d2 < near_lo, b_dh = d2 < dh_lo,
+               b_rep = d2 < rep_lo;
+          const bool edge = valid & ((in != (d2 <= nl_hi)) | (inner != (d2 <= nc_hi)) |
+                                     (b_near != (d2 <= near_hi)) | (b_dh != (d2 <= dh_hi)) |
+                                     (b_rep != (d2 <= rep_hi)));
+          if (__ballot(edge)) {  // the exact FP64 decisions of the pairs in a margin
+            const double dist = pair_dist(k, j);
+            // (what the scan did not count)
+            n_in += __popcll(__ballot(edge & !in & (dist < t_nl)));
+            n_inner += __popcll(__ballot(edge & !inner & (dist < t_nl) & (dist < t_nc)));
+            if (edge) {
+              in = dist < t_nl;
+              inner = in & (dist < t_nc);
+              b_near = !(dist > t_near);
+              b_dh = __ddiv_rn(1.0, dist) > rt_dh;
+              b_rep = dist < t_rep;
+            }
+          }
+          in &= valid;
+          inner &= valid;
+          const bool is_nc = inner & native;
+          bool is4 = false;
+          if (keep4) {
+            const uint32_t wi = csq[k], wj = csq[j];
+            is4 = word_same(wi, wj) & (word_gap(wi, wj) == 4);
+            n_four += __popcll(__ballot(inner & !is_nc & is4));
+          }
+          const bool is_qa = qa_on & inner & !is_nc & (qa4 | !is4);
+          const bool near = is_qa & b_near;
+          const bool rest = in & !is_nc & !is_qa;
+          const bool is_pid = pid_on & rest & inner & (pid4 | !is4);
+          const uint32_t ti = __builtin_bit_cast(uint32_t, pk.w), tj = __builtin_bit_cast(uint32_t, pl.w);
+          const bool is_dh = dh_on & rest & b_dh & (bool)((chg >> (ti & 31)) & (chg >> (tj & 31)) & 1u);
+          const bool is_pauli = pauli_on & rest & b_rep;
+          cnt[RB_NEAR] += __popcll(__ballot(near));
+          cnt[RB_PID] += __popcll(__ballot(is_pid));
+          cnt[RB_DH] += __popcll(__ballot(is_dh));
+          cnt[RB_PAULI] += __popcll(__ballot(is_pauli));
+          const uint32_t cls = (near ? KC_NEAR : 0) | (is_pid ? KC_PID : 0) | (is_dh ? KC_DH : 0) |
+                               (is_pauli ? KC_PAULI : 0);
+          if (valid) kp[t] = word | (cls << 24);
+        }
+        if (!pass) {
+          off[RB_NL] += n_in;
+          // the native contacts among them are taken off once they are counted
+          if (qa_on) off[RB_QA] += n_inner - (qa4 ? 0 : n_four);
+          off[RB_NEAR] += cnt[RB_NEAR];
+          off[RB_PID] += cnt[RB_PID];
+          off[RB_DH] += cnt[RB_DH];
+          off[RB_PAULI] += cnt[RB_PAULI];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
       }
-      continue;
+      if (pass) {
+        // ---- write: each kept pair into its lists at the wave's running
+        // offset plus its rank among the 64's earlier pairs of the list
+        uint32_t next = lane < kept ? kp[lane] : 0u;
+        for (int t0 = 0; t0 < kept; t0 += 64) {
+          const uint32_t word = next;
+          next = t0 + 64 + lane < kept ? kp[t0 + 64 + lane] : 0u;
+          const int k = (int)(word & 0xFFFu), j = (int)((word >> 12) & 0xFFFu);
+          const uint32_t cls = word >> 24;  // 0 past the end
+          const bool near = cls & KC_NEAR, is_pid = cls & KC_PID, is_dh = cls & KC_DH,
+                     is_pauli = cls & KC_PAULI;
+          const int i = r0 + k, jg = r0 + j, ai = g.at[k] & 63, aj = g.at[j] & 63;
+          const u64 m_near = __ballot(near), m_pid = __ballot(is_pid), m_dh = __ballot(is_dh),
+                    m_pauli = __ballot(is_pauli);
+          double d64 = 0.0;
+          if (near | is_pid) d64 = pair_dist(k, j);
+          if (near) {
+            const int fslot = off[RB_NEAR] + rank_in(m_near);
+            if (fslot < sd.qfcap) {
+              const int q = sd.qf0 + fslot;
+              b.qf_i[0][q] = i;
+              b.qf_i[1][q] = jg;
+              b.qf_d[q] = d64;
+              b.qf_vac[q] = 0;
+              // near list entry fslot: the free pair in slot fslot (the
+              // fields only the stage kernels read are left out)
+              const double req = fmax(fmax(fmax(g.req_t[1], g.req_t[2]), g.req_t[3]),
+                                      g.req_t[4 + ai + 21 * aj]);
+              const double thr = fmin(P.qa_max_req, fmax(p.rep_cutoff, req)) * (1.0 + 1e-5);
+              b.qh_slot[q] = fslot;
+              b.qh_thr2[q] = (float)(thr * thr);
+              b.qh_ij[q] = (uint32_t)k | ((uint32_t)j << 16);
+            }
+          }
+          if (is_pid) {
+            const int pos = off[RB_PID] + rank_in(m_pid);
+            if (pos < sd.nlcap) {
+              const int q = sd.nl0 + pos;
+              b.pid_i[0][q] = i;
+              b.pid_i[1][q] = jg;
+              b.pid_d[q] = d64;
+              b.pid_t[q] = (int16_t)(ai * 21 + aj);
+            }
+          }
+          if (is_dh) {
+            const int pos = off[RB_DH] + rank_in(m_dh);
+            if (pos < sd.nlcap) {
+              const int q = sd.nl0 + pos;
+              b.dh_i[0][q] = i;
+              b.dh_i[1][q] = jg;
+              b.dh_q[q] = p.charge[ai] * p.charge[aj];
+            }
+          }
+          if (is_pauli) {
+            const int pos = off[RB_PAULI] + rank_in(m_pauli);
+            if (pos < sd.nlcap) {
+              const int q = sd.nl0 + pos;
+              b.pauli_i[0][q] = i;
+              b.pauli_i[1][q] = jg;
+            }
+          }
+          off[RB_NEAR] += __popcll(m_near);
+          off[RB_PID] += __popcll(m_pid);
+          off[RB_DH] += __popcll(m_dh);
+          off[RB_PAULI] += __popcll(m_pauli);
+        }
+      }
     }
-    for (int k = kbeg; k < kend; ++k) {
-      const double xi = g.x[k], yi = g.y[k], zi = g.z[k];
-      const uint32_t wk = csq[k];
-      const int si = (int)(wk & 0xFFFu), ai = (int)(wk >> 24);
-      const uint32_t ci = (wk >> 12) & 0xFFFu;
-      const int c0 = rs[k], ce = rs[k + 1];
-      int tp = c0;  // the row's next native partner
-      for (int j0 = k + 1; j0 < n; j0 += 64) {
-        const int j = j0 + lane;
-        // native partners among columns j0 .. j0 + 63, as a lane mask
-        unsigned long long natm = 0ull;
-        const int tp0 = tp;
-        while (tp < ce) {
-          const int pt = pj[tp];
-          if (pt > j0 + 63) break;
-          natm |= 1ull << (pt - j0);
-          ++tp;
-        }
-        // straight-line for every lane (column n - 1 stands in for those
-        // past the row's end); the bitwise & and | keep it branch-free
-        const bool valid = j < n;
-        const int jj = valid ? j : n - 1;
-        v3<double> dd = xsub(v3<double>{g.x[jj], g.y[jj], g.z[jj]}, v3<double>{xi, yi, zi});
-        if (cell) dd = xwrapd(dd, sd);
-        const float fx = (float)dd.x, fy = (float)dd.y, fz = (float)dd.z;
-        const float d2 = fx * fx + fy * fy + fz * fz;
-        // columns beyond every threshold and its margin join no list: a
-        // chunk of only such columns adds nothing (its native partners are
-        // already passed)
-        if (!__ballot(valid & (d2 <= e_far))) continue;
-        const uint32_t wj = csq[jj];
-        const int dseq = abs((int)(wj & 0xFFFu) - si);
-        const bool same = ((wj >> 12) & 0xFFFu) == ci;
-        const bool four = same & (dseq == 4);
-        const bool pair = valid & !(same & (dseq < 3));
-        // below a threshold's lower margin the pair is in, above its upper
-        // margin out; between the two (lo != hi) the exact distance decides
-        bool b_nl = d2 < e_nl[0], b_nc = d2 < e_nc[0], b_dh = d2 < e_dh[0], b_rep = d2 < e_rep[0];
-        bool b_near = d2 < e_near[0];
-        const bool edge = pair & ((b_nl != (d2 <= e_nl[1])) | (b_nc != (d2 <= e_nc[1])) |
-                                  (b_dh != (d2 <= e_dh[1])) | (b_rep != (d2 <= e_rep[1])) |
-                                  (b_near != (d2 <= e_near[1])));
-        if (__ballot(edge)) {  // rare: the exact FP64 decisions of the pairs in a band
-          if (edge) {
-            const double dist = xnorm3(dd);
-            b_nl = dist < t_nl;
-            b_nc = dist < t_nc;
-            b_dh = __ddiv_rn(1.0, dist) > rt_dh;
-            b_rep = dist < t_rep;
-            b_near = !(dist > t_near);
-          }
-        }
-        const bool in = pair & b_nl;
-        const bool is_nc = in & b_nc & (bool)((natm >> lane) & 1ull);
-        const bool is_qa = in & !is_nc & qa_on & (qa4 | !four) & b_nc;
-        const bool near = is_qa & b_near;
-        const bool rest = in & !is_nc & !is_qa;
-        const bool is_pid = rest & pid_on & (pid4 | !four) & b_nc;
-        const int aj = (int)(wj >> 24);
-        const bool is_dh = rest & dh_on & (bool)((chg >> ai) & (chg >> aj) & 1u) & b_dh;
-        const bool is_pauli = rest & pauli_on & b_rep;
-        const unsigned long long m_nl = __ballot(in), m_nc = __ballot(is_nc),
-                                 m_qa = __ballot(is_qa), m_near = __ballot(near),
-                                 m_pid = __ballot(is_pid), m_dh = __ballot(is_dh),
-                                 m_pauli = __ballot(is_pauli);
-        if (pass) {
-          const int c = is_nc ? sd.nc0 + tp0 + __popcll(natm & below) : 0;
-          if (valid) emit(k, j, c, is_nc, near, is_pid, is_dh, is_pauli, m_nc, m_near, m_pid,
-                          m_dh, m_pauli, off);
-        } else if (compact) {
-          const bool keep = is_nc | near | is_pid | is_dh | is_pauli;
-          const unsigned long long m_keep = __ballot(keep);
-          if (keep) {
-            const int t = seg + my_nl + __popcll(m_keep & below);
-            b.nl_i[0][t] = (int)((uint32_t)k | ((uint32_t)j << 16));
-            b.nl_cls[t] = (uint8_t)((is_nc ? CL_NC : 0) | (near ? CL_NEAR : 0) |
-                                    (is_pid ? CL_PID : 0) | (is_dh ? CL_DH : 0) |
-                                    (is_pauli ? CL_PAULI : 0));
-            if (is_nc) b.nl_i[1][t] = sd.nc0 + tp0 + __popcll(natm & below);
-          }
-          my_nl += __popcll(m_keep);
-        }
-        off[RB_NL] += __popcll(m_nl);
-        off[RB_NC] += __popcll(m_nc);
-        off[RB_QA] += __popcll(m_qa);
-        off[RB_NEAR] += __popcll(m_near);
-        off[RB_PID] += __popcll(m_pid);
-        off[RB_DH] += __popcll(m_dh);
-        off[RB_PAULI] += __popcll(m_pauli);
+    // ---- the native contacts, each from its own entry of the sorted list: a
+    // wave takes a contiguous run of them, the first pass leaving the mask of
+    // the t-th 64 that are in range in lane t (a wave has fewer than 4096)
+    for (int c0 = cbeg; c0 < cend; c0 += 64) {
+      const int c = min(c0 + lane, cend - 1), turn = (c0 - cbeg) >> 6;
+      u64 m;
+      if (!pass || turn >= 64) {
+        const int i = b.nc_i[0][sd.nc0 + c], jg = b.nc_i[1][sd.nc0 + c];
+        // (a pair listed twice counts once)
+        const bool twice = c > 0 && b.nc_i[0][sd.nc0 + c - 1] == i && b.nc_i[1][sd.nc0 + c - 1] == jg;
+        const uint32_t wi = csq[i - r0], wj = csq[jg - r0];
+        const double dist = pair_dist(i - r0, jg - r0);
+        m = __ballot((c0 + lane < cend) & !twice & (dist < t_nl) & (dist < t_nc) &
+                     !(word_same(wi, wj) & (word_gap(wi, wj) < 3)));
+        if (lane == turn) native_in = m;
+      } else {
+        m = lane_u64(native_in, turn);
       }
+      if (pass && __builtin_amdgcn_inverse_ballot_w64(m))
+        set_current_contact(b, sd.nc0 + off[RB_NC] + rank_in(m), sd.nc0 + c, r0);
+      off[RB_NC] += __popcll(m);
     }
     if (!pass) {
+      if (qa_on) off[RB_QA] -= off[RB_NC];
       if (lane == 0)
         for (int c = 0; c < RB_N; ++c) wcnt[w][c] = off[c];
       __syncthreads();
@@ -468,17 +658,13 @@ __device__ __forceinline__ void wg_fix_nl(DevBatchC *bp, int s, SysState &st, co
     }
   }
   __syncthreads();
-  // the current native contacts' copied fields (set_current_contact), every
-  // slot at once
-  for (int q = threadIdx.x; q < st.nc_n; q += blockDim.x)
-    set_current_contact(b, sd.nc0 + q, b.ncur[sd.nc0 + q], r0);
-  // snapshot (legacy_update.cpp:80-89)
+  // snapshot (legacy_update.cpp:80-89); the force accumulators back to zero
   for (int k = threadIdx.x; k < n; k += blockDim.x) {
     b.orig_r[0][r0 + k] = g.x[k];
     b.orig_r[1][r0 + k] = g.y[k];
     b.orig_r[2][r0 + k] = g.z[k];
+    for (int c = 0; c < 3; ++c) force[c * n + k] = 0.0;
   }
-  __syncthreads();
   if (threadIdx.x == 0) {
     st.orig_pad = pad;
     for (int c = 0; c < 3; ++c) st.orig_cell[c] = sd.cell[c];
@@ -887,7 +1073,8 @@ __device__ __forceinline__ void persistent_body(DevBatchC *bp, int s, int nsteps
   int n, r0, nftip;
   int64_t target;
   bool staged, regular, gear_l, energy_off, nl_required, lang_on;
-  uint32_t on = 0u;  // the enabled terms
+  uint32_t on = 0u;   // the enabled terms
+  uint32_t chg = 0u;  // the residue types with a charge (q1 q2 != 0 iff both are set)
   {
     const DevBatch b = unpack(bp);
     SysDescC &sd = b.sys[s];
@@ -904,6 +1091,7 @@ __device__ __forceinline__ void persistent_body(DevBatchC *bp, int s, int nsteps
     nl_required = P.nl_required != 0;
     lang_on = P.p.lang_on != 0;
     for (int t = 0; t < NT; ++t) on |= (term_on(P, t) ? 1u : 0u) << t;
+    for (int t = 0; t < 21; ++t) chg |= (P.p.charge[t] != 0.0 ? 1u : 0u) << t;
   }
   const bool qa_on = on & (1u << PCG_QA_CAND);
   // forces accumulate in FP64 in LDS: on gfx950 an LDS FP64 atomic add
@@ -978,7 +1166,8 @@ __device__ __forceinline__ void persistent_body(DevBatchC *bp, int s, int nsteps
     if (nl_required) invalid = first || nl_moved(bp, s, st, maxd);
     first = first && !nl_required;
     if (invalid) {
-      wg_fix_nl(bp, s, st, g, (void *)(lds + lay.q));
+      wg_fix_nl(bp, s, st, g, (void *)(lds + lay.q), fx,
+                (float4 *)(lds + ((lay.f + 15) & ~(size_t)15)), chg);
       invalid = false;
     }
     TermTurn turn{0, (int)(blockDim.x >> 6)};
