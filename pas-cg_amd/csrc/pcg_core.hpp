@@ -296,6 +296,7 @@ struct DevBatch {
   int *cell_of, *cell_items, *cell_start, *cell_end;
   int *blk_cnt;               // partition scratch: per-chunk counts
   WallDev *wall;              // plain context: walls and the box protocol (else null)
+  int *ovf;                   // host memory: set when a step ends with an overflow (or null)
 };
 
 // ------------------------------------------------------------- helpers ----

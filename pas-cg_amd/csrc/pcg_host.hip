@@ -362,6 +362,33 @@ struct Arena {
 } // namespace
 
 // A device batch: the systems, their arena and the launch configuration.
+// Pinned host memory that kernels write results into, grown as asked for and
+// kept for the next result of its owner; behind it, the sequence number of the
+// last fetch that has arrived and the overflow flag of the step kernels.
+struct Pinned {
+  char *p = nullptr;
+  size_t cap = 0;
+  int *flag = nullptr, *ovf = nullptr;
+  int seq = 0;
+  int room(size_t bytes) {
+    if (bytes <= cap) return PCG_OK;
+    if (p) HIPCHK(hipHostFree(p));
+    p = nullptr;
+    cap = 0;
+    const size_t want = (bytes + 4095) / 4096 * 4096;
+    HIPCHK(hipHostMalloc((void **)&p, want + 64));
+    cap = want;
+    flag = (int *)(p + cap);
+    ovf = flag + 1;
+    *flag = seq;
+    *ovf = 1;
+    return PCG_OK;
+  }
+  ~Pinned() {
+    if (p) (void)hipHostFree(p);
+  }
+};
+
 struct DeviceBatch {
   int prec = PCG_MIXED;
   int noise = PCG_NOISE_PHILOX;
@@ -379,8 +406,14 @@ struct DeviceBatch {
   int cell_words = 0;  // row-mask words of the largest system on a cell grid
   size_t bytes = 0;
   std::vector<Ran2> ran2;  // per system, RAN2 noise mode
-  std::vector<double> noise_h;
+  // RAN2 noise: a ring of steps' noise in pinned memory and, per slot, the
+  // event after the kernel that reads it
+  static constexpr int NOISE_RING = 8;
   double *noise_pinned = nullptr;
+  hipEvent_t noise_read[NOISE_RING] = {};
+  int noise_at = 0;
+  Pinned own_pin;
+  Pinned *pin = &own_pin;  // a served job's: its server's
   bool own_stream = true;
   // plain context: walls and the box protocol (device copy dW; hW holds its
   // array pointers); box_set once pcg_box_setup ran (the step then runs the
@@ -391,7 +424,10 @@ struct DeviceBatch {
 
   ~DeviceBatch() {
     if (arena.base && !arena.borrowed) (void)hipFree(arena.base);
+    if (noise_pinned && stream) (void)hipStreamSynchronize(stream);
     if (noise_pinned) (void)hipHostFree(noise_pinned);
+    for (hipEvent_t e : noise_read)
+      if (e) (void)hipEventDestroy(e);
     if (stream && own_stream) (void)hipStreamDestroy(stream);
   }
 };
@@ -901,9 +937,33 @@ int make_batch(const pcg_params &p, int nsys, const pcg_model *models, const dou
   return PCG_OK;
 }
 
-int read_state(DeviceBatch &B, int s, SysState &st) {
-  HIPCHK(hipMemcpyAsync(&st, B.d.st + s, sizeof(SysState), hipMemcpyDeviceToHost, B.stream));
+// Enqueues a fetch into the batch's pinned memory (its room already made) and
+// waits for it to arrive: the host reads the flag for a while, which a fetch
+// behind idle work raises within some microseconds, then waits for the stream.
+int fetch_now(DeviceBatch &B, Fetch f) {
+  Pinned &pin = *B.pin;
+  f.flag = pin.flag;
+  f.seq = ++pin.seq;
+  launch_fetch(f, B.stream);
+  HIPCHK(hipGetLastError());
+  for (int spin = 0; spin < 20000; ++spin) {
+    if (__atomic_load_n(pin.flag, __ATOMIC_ACQUIRE) == f.seq) return PCG_OK;
+    __builtin_ia32_pause();
+  }
   HIPCHK(hipStreamSynchronize(B.stream));
+  return PCG_OK;
+}
+int read_state(DeviceBatch &B, int s, SysState &st) {
+  static_assert(sizeof(SysState) % 4 == 0, "fetched as words");
+  HIPCHK(hipSetDevice(B.device));
+  Fetch f;
+  f.bytes = sizeof(SysState);
+  int rc = B.pin->room(f.bytes);
+  if (rc) return rc;
+  f.src = B.d.st + s;
+  f.dst = B.pin->p;
+  if ((rc = fetch_now(B, f))) return rc;
+  std::memcpy(&st, B.pin->p, sizeof(SysState));
   return PCG_OK;
 }
 int write_state(DeviceBatch &B, int s, const SysState &st) {
@@ -912,56 +972,47 @@ int write_state(DeviceBatch &B, int s, const SysState &st) {
   return PCG_OK;
 }
 
-// copies 3 device columns of system s into xyz-interleaved host memory
-int get_cols(DeviceBatch &B, int s, double *const cols[3], double *out) {
-  const SysDesc &d = B.sys[s];
-  std::vector<double> tmp(3 * (size_t)d.n);
+// A fetch of three device columns of system s (FP32 or FP64) to byte `at` of
+// the batch's pinned memory, as FP64 triples.
+Fetch fetch_of(DeviceBatch &B, int s, const void *const cols[3], bool f32, size_t at) {
+  Fetch f;
   for (int c = 0; c < 3; ++c)
-    HIPCHK(hipMemcpyAsync(tmp.data() + c * d.n, cols[c] + d.res0, d.n * 8, hipMemcpyDeviceToHost,
-                          B.stream));
-  HIPCHK(hipStreamSynchronize(B.stream));
-  for (int i = 0; i < d.n; ++i)
-    for (int c = 0; c < 3; ++c) out[3 * i + c] = tmp[c * d.n + i];
+    f.cols[c] = (const char *)cols[c] + (size_t)(f32 ? 4 : 8) * B.sys[s].res0;
+  f.f32 = f32;
+  f.n = B.sys[s].n;
+  f.out = (double *)(B.pin->p + at);
+  return f;
+}
+// 3 device columns of system s into xyz-interleaved host memory
+int get_triples(DeviceBatch &B, int s, const void *const cols[3], bool f32, double *out) {
+  const size_t bytes = 24 * (size_t)B.sys[s].n;
+  HIPCHK(hipSetDevice(B.device));
+  int rc = B.pin->room(bytes);
+  if (rc || (rc = fetch_now(B, fetch_of(B, s, cols, f32, 0)))) return rc;
+  std::memcpy(out, B.pin->p, bytes);
   return PCG_OK;
 }
+int get_cols(DeviceBatch &B, int s, double *const cols[3], double *out) {
+  const void *c[3] = {cols[0], cols[1], cols[2]};
+  return get_triples(B, s, c, false, out);
+}
 int get_forces(DeviceBatch &B, int s, double *out) {
-  const SysDesc &d = B.sys[s];
-  size_t fsz = B.prec == PCG_FP64 ? 8 : 4;
-  std::vector<char> tmp(3 * fsz * d.n);
-  for (int c = 0; c < 3; ++c)
-    HIPCHK(hipMemcpyAsync(tmp.data() + c * fsz * d.n, (char *)B.d.F[c] + fsz * d.res0, fsz * d.n,
-                          hipMemcpyDeviceToHost, B.stream));
-  HIPCHK(hipStreamSynchronize(B.stream));
-  for (int i = 0; i < d.n; ++i)
-    for (int c = 0; c < 3; ++c)
-      out[3 * i + c] = B.prec == PCG_FP64 ? ((double *)tmp.data())[c * d.n + i]
-                                          : (double)((float *)tmp.data())[c * d.n + i];
-  return PCG_OK;
+  return get_triples(B, s, B.d.F, B.prec != PCG_FP64, out);
 }
 
 // The same three columns to or from caller arrays of one component each,
-// element i at comp[c][i * stride]; unit stride copies straight between the
-// device columns and the caller's arrays.
+// element i at comp[c][i * stride].
+void spread3(const double *triples, int n, double *const out[3], int64_t stride) {
+  for (int i = 0; i < n; ++i)
+    for (int c = 0; c < 3; ++c) out[c][(size_t)i * stride] = triples[3 * (size_t)i + c];
+}
 int get_cols3(DeviceBatch &B, int s, const void *const cols[3], bool f32, double *const out[3],
               int64_t stride) {
-  const SysDesc &d = B.sys[s];
-  const size_t esz = f32 ? 4 : 8;
-  if (stride == 1 && !f32) {
-    for (int c = 0; c < 3; ++c)
-      HIPCHK(hipMemcpyAsync(out[c], (const char *)cols[c] + esz * d.res0, d.n * esz,
-                            hipMemcpyDeviceToHost, B.stream));
-    HIPCHK(hipStreamSynchronize(B.stream));
-    return PCG_OK;
-  }
-  std::vector<char> tmp(3 * esz * d.n);
-  for (int c = 0; c < 3; ++c)
-    HIPCHK(hipMemcpyAsync(tmp.data() + c * esz * d.n, (const char *)cols[c] + esz * d.res0,
-                          esz * d.n, hipMemcpyDeviceToHost, B.stream));
-  HIPCHK(hipStreamSynchronize(B.stream));
-  for (int c = 0; c < 3; ++c)
-    for (int i = 0; i < d.n; ++i)
-      out[c][(size_t)i * stride] = f32 ? (double)((const float *)tmp.data())[c * d.n + i]
-                                       : ((const double *)tmp.data())[c * d.n + i];
+  const int n = B.sys[s].n;
+  HIPCHK(hipSetDevice(B.device));
+  int rc = B.pin->room(24 * (size_t)n);
+  if (rc || (rc = fetch_now(B, fetch_of(B, s, cols, f32, 0)))) return rc;
+  spread3((const double *)B.pin->p, n, out, stride);
   return PCG_OK;
 }
 int set_cols3(DeviceBatch &B, int s, double *const cols[3], const double *const in[3],
@@ -984,20 +1035,28 @@ int set_cols3(DeviceBatch &B, int s, double *const cols[3], const double *const 
 }
 
 // Reference-order noise for RAN2 mode: all x, then all y, then all z per
-// system (cg/src/cg/langevin/step.cpp:119-127).
+// system (cg/src/cg/langevin/step.cpp:119-127). The host draws a step's noise
+// into the next slot of the ring while the device runs the steps before; it
+// waits only for the kernel that read that slot NOISE_RING steps ago.
 int upload_ran2_noise(DeviceBatch &B) {
-  int ntot = B.d.ntot;
-  if (!B.noise_pinned) HIPCHK(hipHostMalloc((void **)&B.noise_pinned, 3 * ntot * sizeof(double)));
+  const size_t ntot = B.d.ntot;
+  if (!B.noise_pinned) {
+    HIPCHK(hipHostMalloc((void **)&B.noise_pinned,
+                         DeviceBatch::NOISE_RING * 3 * ntot * sizeof(double)));
+    for (hipEvent_t &e : B.noise_read) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
+  const int slot = B.noise_at;
+  B.noise_at = (slot + 1) % DeviceBatch::NOISE_RING;
+  HIPCHK(hipEventSynchronize(B.noise_read[slot]));  // (complete if never recorded)
+  double *nz = B.noise_pinned + slot * 3 * ntot;
   for (size_t s = 0; s < B.sys.size(); ++s) {
     const SysDesc &d = B.sys[s];
     for (int c = 0; c < 3; ++c)
-      for (int i = 0; i < d.n; ++i) B.noise_pinned[c * ntot + d.res0 + i] = B.ran2[s].normal();
+      for (int i = 0; i < d.n; ++i) nz[c * ntot + d.res0 + i] = B.ran2[s].normal();
   }
-  for (int c = 0; c < 3; ++c)
-    HIPCHK(hipMemcpyAsync(B.d.noise[c], B.noise_pinned + c * ntot, ntot * 8, hipMemcpyHostToDevice,
-                          B.stream));
-  // the pinned buffer is rewritten next step: wait for the copy
-  HIPCHK(hipStreamSynchronize(B.stream));
+  launch_noise_in(B.d, nz, B.stream);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipEventRecord(B.noise_read[slot], B.stream));
   return PCG_OK;
 }
 
@@ -1171,12 +1230,18 @@ int report_into_static(DeviceBatch &B, double *out) {
 }
 
 int check_overflow(DeviceBatch &B) {
-  // every system's scalars in one copy
-  std::vector<SysState> st(B.sys.size());
-  HIPCHK(hipMemcpyAsync(st.data(), B.d.st, st.size() * sizeof(SysState), hipMemcpyDeviceToHost,
-                        B.stream));
-  HIPCHK(hipStreamSynchronize(B.stream));
-  for (size_t s = 0; s < st.size(); ++s)
+  // every system's scalars at once
+  const size_t ns = B.sys.size();
+  HIPCHK(hipSetDevice(B.device));
+  int rc = B.pin->room(ns * sizeof(SysState));
+  if (rc) return rc;
+  Fetch f;
+  f.src = B.d.st;
+  f.dst = B.pin->p;
+  f.bytes = ns * sizeof(SysState);
+  if ((rc = fetch_now(B, f))) return rc;
+  const SysState *st = (const SysState *)B.pin->p;
+  for (size_t s = 0; s < ns; ++s)
     if (st[s].overflow)
       return fail(PCG_E_OVERFLOW, "a neighbour or QA list of system " + std::to_string(s) +
                                       " outgrew its capacity");
@@ -1190,6 +1255,27 @@ int check_overflow(DeviceBatch &B) {
                                   "outgrew their capacity");
   }
   return PCG_OK;
+}
+// The overflow flag the step kernels raise in host memory, set up before the
+// first launch. It starts (and, after a restored state, is put back) raised,
+// so the states themselves are looked at once; then steps that end without an
+// overflow cost the host one read of it.
+// (The memory is made for the largest result of the batch here: it never
+// moves afterwards, so captured launches keep the flag's address.)
+int watch_overflow(DeviceBatch &B) {
+  const size_t triples = 24 * (size_t)B.max_n + 1024, states = B.sys.size() * sizeof(SysState);
+  int rc = B.own_pin.room(std::max(triples, states));
+  if (rc) return rc;
+  B.d.ovf = B.own_pin.ovf;
+  return PCG_OK;
+}
+// check_overflow at the end of complete steps, the stream idle
+int check_step_overflow(DeviceBatch &B) {
+  volatile int *flag = B.d.ovf;
+  if (flag && !*flag && !(B.dW && B.hp.ljw_terms)) return PCG_OK;
+  const int rc = check_overflow(B);
+  if (flag && rc == PCG_OK) *flag = 0;
+  return rc;
 }
 
 // Whether the lean kernels (LEAN in pcg_persist.hpp) carry everything this
@@ -1291,14 +1377,6 @@ void enqueue_step(DeviceBatch &B) {
   launch_lang(d, B.prec, B.noise, B.stream, true);
 }
 
-// the reaction forces of the walls start a term evaluation at zero
-int zero_wall_F(DeviceBatch &B) {
-  if (B.dW)
-    HIPCHK(hipMemsetAsync((char *)B.dW + offsetof(WallDev, wall_F), 0, sizeof(B.hW.wall_F),
-                          B.stream));
-  return PCG_OK;
-}
-
 // the host copy of the system descriptor after the box protocol moved the
 // PBC cell on the device
 int refresh_sys(DeviceBatch &B) {
@@ -1376,6 +1454,7 @@ int pcg_create(const pcg_params *p, const pcg_model *m, const pcg_options *o, pc
                       nullptr, nullptr, opt.ran2_skip, nullptr, 0, true);
   if (rc) return rc;
   c->B->noise = opt.noise;
+  if ((rc = watch_overflow(*c->B))) return rc;
   {
     DeviceBatch &B = *c->B;
     c->pcfg = persistent_cfg(B);
@@ -1414,7 +1493,7 @@ int pcg_step(pcg_ctx *c, int32_t nsteps) {
                         c->pcfg.lds, B.stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(B.stream));
-    return check_overflow(B);
+    return check_step_overflow(B);
   }
   if ((rc = switch_form(*c, FORM_STAGES))) return rc;
   for (int k = 0; k < nsteps; ++k) {
@@ -1432,7 +1511,7 @@ int pcg_step(pcg_ctx *c, int32_t nsteps) {
     }
   }
   HIPCHK(hipStreamSynchronize(B.stream));
-  return check_overflow(B);
+  return check_step_overflow(B);
 }
 
 int pcg_use_graph(pcg_ctx *c, int32_t on) {
@@ -1468,15 +1547,11 @@ int pcg_nl_verify(pcg_ctx *c, int32_t *invalid) {
 int pcg_fix_nl(pcg_ctx *c) {
   if (!c) return fail(PCG_E_ARG, "null ctx");
   DeviceBatch &B = *c->B;
-  SysState st;
+  HIPCHK(hipSetDevice(B.device));
   int rc = switch_form(*c, FORM_STAGES);
-  if (rc || (rc = read_state(B, 0, st))) return rc;
   if (rc) return rc;
-  st.nl_invalid = 1;
-  st.verify_first = 0;
-  if ((rc = write_state(B, 0, st))) return rc;
+  launch_mark_invalid(B.d, B.stream);
   launch_fix_nl(B.d, B.max_n, B.max_nlcap, B.cell_words, B.stream);
-  HIPCHK(hipStreamSynchronize(B.stream));
   return check_overflow(B);
 }
 
@@ -1492,17 +1567,12 @@ int pcg_prepare_nh(pcg_ctx *c) {
 int pcg_eval_forces(pcg_ctx *c) {
   if (!c) return fail(PCG_E_ARG, "null ctx");
   DeviceBatch &B = *c->B;
-  SysState st;
+  HIPCHK(hipSetDevice(B.device));
   int rc = switch_form(*c, FORM_STAGES);
-  if (rc || (rc = read_state(B, 0, st))) return rc;
   if (rc) return rc;
-  for (int k = 0; k < NT; ++k) st.V[k] = 0.0;
-  if ((rc = write_state(B, 0, st))) return rc;
-  if ((rc = zero_wall_F(B))) return rc;
-  launch_zero_forces(B.d, B.prec, B.stream);
+  launch_eval_begin(B.d, B.prec, B.stream);
   launch_terms(B.d, B.prec, B.max_items, -1, 0, -1, B.stream);
   launch_tick(B.d, 0, B.stream);
-  HIPCHK(hipStreamSynchronize(B.stream));
   return check_overflow(B);
 }
 
@@ -1542,44 +1612,58 @@ int pcg_term_size(pcg_ctx *c, int32_t term, int32_t *size) {
   return PCG_OK;
 }
 
-static int eval_term_only(pcg_ctx *c, int32_t term, int32_t from, int32_t to, double *V) {
+// One term, its forces as triples (want_F) and the state after it in pinned
+// memory behind one wait; the triples at *F, the energy in V.
+static int eval_term_only(pcg_ctx *c, int32_t term, int32_t from, int32_t to, bool want_F,
+                          const double **F, double *V) {
   if (!c || term < 0 || term >= NT) return fail(PCG_E_ARG, "bad arguments");
   DeviceBatch &B = *c->B;
-  SysState st;
   int rc = switch_form(*c, FORM_STAGES);
-  if (rc || (rc = read_state(B, 0, st))) return rc;
   if (rc) return rc;
-  for (int k = 0; k < NT; ++k) st.V[k] = 0.0;
-  if ((rc = write_state(B, 0, st))) return rc;
-  if ((rc = zero_wall_F(B))) return rc;
-  launch_zero_forces(B.d, B.prec, B.stream);
+  HIPCHK(hipSetDevice(B.device));
+  const size_t at = (sizeof(SysState) + 255) / 256 * 256;
+  if ((rc = B.pin->room(at + (want_F ? 24 * (size_t)B.sys[0].n : 0)))) return rc;
+  launch_eval_begin(B.d, B.prec, B.stream);
   launch_terms(B.d, B.prec, B.max_items, term, from, to, B.stream);
-  HIPCHK(hipStreamSynchronize(B.stream));
-  if ((rc = read_state(B, 0, st))) return rc;
+  Fetch f;
+  if (want_F) f = fetch_of(B, 0, B.d.F, B.prec != PCG_FP64, at);
+  f.src = B.d.st;
+  f.dst = B.pin->p;
+  f.bytes = sizeof(SysState);
+  if ((rc = fetch_now(B, f))) return rc;
+  const SysState &st = *(const SysState *)B.pin->p;
   if (V) *V = st.V[term];
+  *F = (const double *)(B.pin->p + at);
   return PCG_OK;
+}
+// the state of the last eval_term_only holds no overflow (else the full check
+// words the error); the walls' lists are looked at themselves
+static int eval_term_check(pcg_ctx *c) {
+  DeviceBatch &B = *c->B;
+  if (!((const SysState *)B.pin->p)->overflow && !(B.dW && B.hp.ljw_terms)) return PCG_OK;
+  return check_overflow(B);
 }
 
 int pcg_eval_term(pcg_ctx *c, int32_t term, int32_t from, int32_t to, double *F, double *V) {
-  int rc = eval_term_only(c, term, from, to, V);
+  const double *triples;
+  int rc = eval_term_only(c, term, from, to, F != nullptr, &triples, V);
   if (rc) return rc;
-  if (F && (rc = get_forces(*c->B, 0, F))) return rc;
-  return check_overflow(*c->B);
+  if (F) std::memcpy(F, triples, 24 * (size_t)c->B->sys[0].n);
+  return eval_term_check(c);
 }
 
 int pcg_eval_term3(pcg_ctx *c, int32_t term, int32_t from, int32_t to, double *Fx, double *Fy,
                    double *Fz, int64_t stride, double *V) {
   if ((Fx || Fy || Fz) && (!Fx || !Fy || !Fz || stride < 1))
     return fail(PCG_E_ARG, "pcg_eval_term3: all three components and a positive stride");
-  int rc = eval_term_only(c, term, from, to, V);
+  const double *triples;
+  int rc = eval_term_only(c, term, from, to, Fx != nullptr, &triples, V);
   if (rc) return rc;
-  DeviceBatch &B = *c->B;
   if (Fx) {
-    const void *cols[3] = {B.d.F[0], B.d.F[1], B.d.F[2]};
     double *const out[3] = {Fx, Fy, Fz};
-    if ((rc = get_cols3(B, 0, cols, B.prec != PCG_FP64, out, stride))) return rc;
+    spread3(triples, c->B->sys[0].n, out, stride);
   }
-  return check_overflow(B);
+  return eval_term_check(c);
 }
 
 int pcg_qa_finish(pcg_ctx *c) {
@@ -1587,7 +1671,6 @@ int pcg_qa_finish(pcg_ctx *c) {
   int rc = switch_form(*c, FORM_STAGES);
   if (rc) return rc;
   launch_qa_finish(c->B->d, c->B->max_n, c->B->stream);
-  HIPCHK(hipStreamSynchronize(c->B->stream));
   return check_overflow(*c->B);
 }
 
@@ -1939,6 +2022,7 @@ int pcg_batch_create(const pcg_params *p, int32_t nsys, const pcg_model *models,
                       b->B);
   if (rc) return rc;
   DeviceBatch &B = *b->B;
+  if ((rc = watch_overflow(B))) return rc;
   // per-residue bonded data joins positions and forces in LDS when it fits;
   // systems whose positions and forces do not fit take the stage kernels
   const PersistentCfg pc = persistent_cfg(B);
@@ -1972,7 +2056,7 @@ int pcg_batch_run(pcg_batch *b, int32_t nsteps) {
   HIPCHK(hipSetDevice(b->B->device));
   int rc = b->persistent ? run_persistent(b, nsteps) : run_stages(b, nsteps);
   if (rc) return rc;
-  return check_overflow(*b->B);
+  return check_step_overflow(*b->B);
 }
 
 int pcg_batch_sync(pcg_batch *b) {
@@ -2119,6 +2203,7 @@ int ckpt_read(DeviceBatch &B, const char magic[8], const void *buf, int64_t byte
   HIPCHK(hipMemcpyAsync(B.sys.data(), (const void *)B.d.sys, B.sys.size() * sizeof(SysDesc),
                         hipMemcpyDeviceToHost, B.stream));
   HIPCHK(hipStreamSynchronize(B.stream));
+  if (B.d.ovf) *B.d.ovf = 1;
   if (!B.ran2.empty())
     std::memcpy(B.ran2.data(), (const char *)buf + sizeof h + B.arena.total,
                 B.ran2.size() * sizeof(Ran2));
@@ -2614,6 +2699,7 @@ struct pcg_server {
   std::multimap<size_t, void *> pool;
   size_t pooled_bytes = 0;
   double noise_scale = 1.0;  // scales the Langevin noise of every job
+  Pinned pin;                // every job's results come back through it
   ~pcg_server() {
     for (auto &bk : bucket)
       if (bk.stream) (void)hipStreamSynchronize(bk.stream);
@@ -2645,15 +2731,25 @@ int retire(pcg_server *s, Job &j, int status) {
   if (j.B) {
     SysState st;
     if (status == PCG_JOB_DONE) {
-      const size_t n3 = 3 * (size_t)j.model.n;
-      j.result.assign(n3, 0.0);
-      j.result_F.assign(n3, 0.0);
-      j.result_vel.assign(n3, 0.0);
-      int rc = get_cols(*j.B, 0, j.B->d.y[0], j.result.data());
+      // positions, forces, velocities and the state behind one wait
+      DeviceBatch &B = *j.B;
+      const size_t n3 = 3 * (size_t)j.model.n, col = 8 * n3;
+      int rc = B.pin->room(3 * col + sizeof(SysState));
       if (rc) return rc;
-      if ((rc = get_forces(*j.B, 0, j.result_F.data()))) return rc;
-      if ((rc = get_cols(*j.B, 0, j.B->d.vel, j.result_vel.data()))) return rc;
-      if ((rc = read_state(*j.B, 0, st))) return rc;
+      const void *y0[3] = {B.d.y[0][0], B.d.y[0][1], B.d.y[0][2]};
+      const void *vel[3] = {B.d.vel[0], B.d.vel[1], B.d.vel[2]};
+      launch_fetch(fetch_of(B, 0, y0, false, 0), B.stream);
+      launch_fetch(fetch_of(B, 0, B.d.F, B.prec != PCG_FP64, col), B.stream);
+      Fetch f = fetch_of(B, 0, vel, false, 2 * col);
+      f.src = B.d.st;
+      f.dst = B.pin->p + 3 * col;
+      f.bytes = sizeof(SysState);
+      if ((rc = fetch_now(B, f))) return rc;
+      const double *got = (const double *)B.pin->p;
+      j.result.assign(got, got + n3);
+      j.result_F.assign(got + n3, got + 2 * n3);
+      j.result_vel.assign(got + 2 * n3, got + 3 * n3);
+      std::memcpy(&st, B.pin->p + 3 * col, sizeof(SysState));
       j.V = st.Vtot;
       j.done = st.step;
     }
@@ -2898,6 +2994,7 @@ int serve_admit(pcg_server *s) {
                             bk.stream));
     }
     j.B->lean = lean_batch(*j.B);
+    j.B->pin = &s->pin;
     j.status = PCG_JOB_RUNNING;
     j.t_start = now_s();
     j.block_bytes = blk_bytes;

@@ -44,13 +44,54 @@ __global__ void k_begin(DevBatch b) {
   begin_system(b, s);
 }
 
-template <typename RF> __global__ void k_zero_forces(DevBatch b) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+// Before an evaluation outside a step: forces, energies and the walls'
+// reaction forces at zero.
+template <typename RF> __global__ void k_eval_begin(DevBatch b) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= b.ntot) return;
-  if (!b.st[b.sysid[i]].active) return;
-  ((RF *)b.F[0])[i] = 0;
-  ((RF *)b.F[1])[i] = 0;
-  ((RF *)b.F[2])[i] = 0;
+  const int s = b.sysid[i];
+  if (b.local[i] == 0) {
+    for (int k = 0; k < NT; ++k) b.st[s].V[k] = 0.0;
+    if (b.wall)
+      for (int w = 0; w < 6; ++w)
+        for (int c = 0; c < 3; ++c) b.wall->wall_F[w][c] = 0.0;
+  }
+  if (!b.st[s].active) return;
+  for (int c = 0; c < 3; ++c) ((RF *)b.F[c])[i] = 0;
+}
+
+// The next rebuild of every system is due.
+__global__ void k_mark_invalid(DevBatch b) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= b.nsys) return;
+  b.st[s].nl_invalid = 1;
+  b.st[s].verify_first = 0;
+}
+
+// Device data into mapped pinned host memory: words as they are, and three
+// columns as interleaved FP64 triples; one workgroup, which then writes seq to
+// the host's flag, so that the host sees the result arrive by reading the flag
+// instead of waiting for the stream (9 us a call for a system's positions;
+// 14 us with a wait for the stream, 47 us as three staged column copies).
+template <typename T>
+__global__ __launch_bounds__(1024) void k_fetch(const uint32_t *words, uint32_t *words_out, int nw,
+                                                const T *x, const T *y, const T *z, double *out,
+                                                int n, int *flag, int seq) {
+  for (int i = threadIdx.x; i < nw; i += blockDim.x) words_out[i] = words[i];
+  for (int i = threadIdx.x; i < 3 * n; i += blockDim.x) {
+    const int k = i / 3, c = i - 3 * k;
+    out[i] = (double)(c == 0 ? x : c == 1 ? y : z)[k];
+  }
+  if (!flag) return;
+  // every wave's stores are out before the barrier; one release covers them
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// the host's noise for one step (ntot x, then y, then z) into the device's
+__global__ void k_noise_in(DevBatch b, const double *src) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= b.ntot) return;
+  for (int c = 0; c < 3; ++c) b.noise[c][i] = src[(size_t)c * b.ntot + i];
 }
 
 // ------------------------------------------------------------ NL rebuild ----
@@ -593,7 +634,7 @@ __global__ void k_prepare_nh(DevBatch b) {
 // The first kernel of a full step, over residues: each system's first
 // residue runs the system's begin (energies and the walls' reaction forces
 // cleared, nl::verify), every residue clears its force and, with QA on,
-// computes its n and h (k_begin, k_zero_forces and k_prepare_nh in one
+// computes its n and h (k_begin, the force clearing and k_prepare_nh in one
 // launch; none reads what another writes)
 template <typename RF> __global__ void k_step_begin(DevBatch b, int qa_on) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -656,6 +697,7 @@ __device__ __forceinline__ void tick_system(const DevBatch &b, int s, int advanc
   double v = 0.0;
   for (int k = 0; k < NT; ++k) v += st.V[k];
   st.Vtot = v;
+  if (b.ovf && st.overflow) *b.ovf = 1;
   if (advance && b.P->p.lang_on) {
     st.true_t += b.P->dt;
     st.t = st.true_t;
@@ -1073,11 +1115,30 @@ static inline dim3 grid1(int n, int blk = BLK) { return dim3((unsigned)((n + blk
 void launch_begin(const DevBatch &b, hipStream_t s) {
   hipLaunchKernelGGL(k_begin, grid1(b.nsys, 64), dim3(64), 0, s, b);
 }
-void launch_zero_forces(const DevBatch &b, int prec, hipStream_t s) {
+void launch_eval_begin(const DevBatch &b, int prec, hipStream_t s) {
   if (prec == PCG_FP64)
-    hipLaunchKernelGGL(k_zero_forces<double>, grid1(b.ntot), dim3(BLK), 0, s, b);
+    hipLaunchKernelGGL(k_eval_begin<double>, grid1(b.ntot), dim3(BLK), 0, s, b);
   else
-    hipLaunchKernelGGL(k_zero_forces<float>, grid1(b.ntot), dim3(BLK), 0, s, b);
+    hipLaunchKernelGGL(k_eval_begin<float>, grid1(b.ntot), dim3(BLK), 0, s, b);
+}
+void launch_mark_invalid(const DevBatch &b, hipStream_t s) {
+  hipLaunchKernelGGL(k_mark_invalid, grid1(b.nsys, 64), dim3(64), 0, s, b);
+}
+void launch_fetch(const Fetch &f, hipStream_t s) {
+  const int most = std::max((int)(f.bytes / 4), 3 * f.n);
+  const dim3 block((unsigned)std::min(1024, std::max(64, (most + 63) / 64 * 64)));
+  if (f.f32)
+    hipLaunchKernelGGL(k_fetch<float>, dim3(1), block, 0, s, (const uint32_t *)f.src,
+                       (uint32_t *)f.dst, (int)(f.bytes / 4), (const float *)f.cols[0],
+                       (const float *)f.cols[1], (const float *)f.cols[2], f.out, f.n, f.flag, f.seq);
+  else
+    hipLaunchKernelGGL(k_fetch<double>, dim3(1), block, 0, s, (const uint32_t *)f.src,
+                       (uint32_t *)f.dst, (int)(f.bytes / 4), (const double *)f.cols[0],
+                       (const double *)f.cols[1], (const double *)f.cols[2], f.out, f.n, f.flag,
+                       f.seq);
+}
+void launch_noise_in(const DevBatch &b, const double *src, hipStream_t s) {
+  hipLaunchKernelGGL(k_noise_in, grid1(b.ntot), dim3(BLK), 0, s, b, src);
 }
 void launch_prepare_nh(const DevBatch &b, hipStream_t s) {
   hipLaunchKernelGGL(k_prepare_nh, grid1(b.ntot), dim3(BLK), 0, s, b);

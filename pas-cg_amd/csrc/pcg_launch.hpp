@@ -5,7 +5,25 @@
 
 namespace pcg {
 void launch_begin(const DevBatch &b, hipStream_t s);
-void launch_zero_forces(const DevBatch &b, int prec, hipStream_t s);
+// forces, energies and wall reactions to zero before an evaluation outside a step
+void launch_eval_begin(const DevBatch &b, int prec, hipStream_t s);
+void launch_mark_invalid(const DevBatch &b, hipStream_t s);
+// device data into mapped pinned host memory: bytes of src as words, and three
+// columns of n values (FP32 or FP64) as FP64 triples; then seq into flag
+struct Fetch {
+  const void *src = nullptr;
+  void *dst = nullptr;
+  size_t bytes = 0;
+  const void *cols[3] = {nullptr, nullptr, nullptr};
+  bool f32 = false;
+  int n = 0;
+  double *out = nullptr;
+  int *flag = nullptr;  // null: no flag
+  int seq = 0;
+};
+void launch_fetch(const Fetch &f, hipStream_t s);
+// the host's noise of one step into the device's
+void launch_noise_in(const DevBatch &b, const double *src, hipStream_t s);
 void launch_prepare_nh(const DevBatch &b, hipStream_t s);
 // begin, force clearing and (qa_on) prepare_nh of a full step in one launch
 void launch_step_begin(const DevBatch &b, int prec, int qa_on, hipStream_t s);

@@ -1295,6 +1295,7 @@ __device__ __forceinline__ void persistent_body(DevBatchC *bp, int s, int nsteps
       st.Vtot = v;
     }
     b.st[s] = st;
+    if (b.ovf && st.overflow) *b.ovf = 1;
     if (slot) {
       slot->step = st.step;
       slot->Vtot = st.Vtot;
