@@ -15,7 +15,7 @@
 namespace pcg {
 
 constexpr int NT = PCG_NUM_TERMS;
-// partition classes of an NL pair in the stage kernels (per-chunk counts)
+// (sizes blk_cnt)
 constexpr int NCL = 6;
 // Static bonded lists whose items are chain-local: item of base residue r
 // spans r, r+1 (tether), r, r+2 (local repulsion), r..r+2 (angles) or
@@ -233,6 +233,7 @@ struct DevBatch {
   double *y[6][3];            // Gear y0..y5 (y0 = positions)
   double *vel[3];
   void *F[3];                 // float or double forces (precision)
+  double *acc[3];             // stage kernels: the forces' FP64 accumulators (F itself in FP64)
   double *orig_r[3];          // positions at the last NL rebuild
   double *nat_r[3];           // the model's original positions (the report's RMSD reference)
   double *nh[6];              // QA n and h vectors (FP64)
@@ -253,7 +254,7 @@ struct DevBatch {
   const int *tip_res; const double *tip_orig[3], *tip_vel[3];
   TipStat *tip_stat;          // per tip slot, as tip_res
   // dynamic lists
-  int *nl_i[2]; double *nl_d; uint8_t *nl_cls;  // class bits of the partition
+  int *nl_i[2]; double *nl_d; uint8_t *nl_cls;  // unused: saved states have room for it
   int *ncur;                                      // current native contacts (index into all)
   int *ncur_i[2]; double *ncur_nat;  // their residues, length,
   uint8_t *ncur_t;                   // type | active << 7
@@ -294,7 +295,7 @@ struct DevBatch {
   // (system-local indices), each cell's first slot and its end (a count
   // between the rebuild's kernels, zero between rebuilds)
   int *cell_of, *cell_items, *cell_start, *cell_end;
-  int *blk_cnt;               // partition scratch: per-chunk counts
+  int *blk_cnt;               // unused: saved states have room for it
   WallDev *wall;              // plain context: walls and the box protocol (else null)
   int *ovf;                   // host memory: set when a step ends with an overflow (or null)
 };

@@ -400,7 +400,7 @@ struct DeviceBatch {
   std::vector<SysDesc> sys;
   std::vector<HostSys> hs;
   Arena arena;
-  int max_nlcap = 0, max_n = 0, max_items = 0;
+  int max_n = 0, max_items = 0;
   int max_nnc = 0;  // most native contacts of one system
   bool lean = false;  // served job: the lean kernels carry it (once staged)
   int cell_words = 0;  // row-mask words of the largest system on a cell grid
@@ -421,8 +421,10 @@ struct DeviceBatch {
   WallDev *dW = nullptr;
   WallDev hW{};
   bool box_set = false;
+  double *acc = nullptr;  // stage kernels, mixed precision: DevBatch::acc
 
   ~DeviceBatch() {
+    if (acc) (void)hipFree(acc);
     if (arena.base && !arena.borrowed) (void)hipFree(arena.base);
     if (noise_pinned && stream) (void)hipStreamSynchronize(stream);
     if (noise_pinned) (void)hipHostFree(noise_pinned);
@@ -533,7 +535,6 @@ int make_batch(const pcg_params &p, int nsys, const pcg_model *models, const dou
     nteth += d.nteth, nlrep += d.nlrep, nchir += d.nchir, nnang += d.nnang, nhang += d.nhang;
     nndih += d.nndih, nhdih += d.nhdih, nnc += d.nnc, ntip += d.ntip + d.nftip;
     nl += h.nlcap, qf += h.qfcap, qc += h.qccap;
-    B->max_nlcap = std::max(B->max_nlcap, h.nlcap);
     B->max_n = std::max(B->max_n, h.n);
     B->max_nnc = std::max(B->max_nnc, d.nnc);
     int items = std::max({d.nteth, d.nlrep, d.nchir, d.nnang, d.nhang, d.nndih, d.nhdih, d.nnc,
@@ -1269,6 +1270,15 @@ int watch_overflow(DeviceBatch &B) {
   B.d.ovf = B.own_pin.ovf;
   return PCG_OK;
 }
+// The stage kernels' force accumulators: FP64 in every precision, so in mixed
+// precision apart from the force arrays.
+int stage_forces(DeviceBatch &B) {
+  const size_t n = B.d.ntot;
+  if (B.prec != PCG_FP64) HIPCHK(hipMalloc((void **)&B.acc, 3 * n * sizeof(double)));
+  for (int c = 0; c < 3; ++c) B.d.acc[c] = B.acc ? B.acc + c * n : (double *)B.d.F[c];
+  if (B.acc) B.bytes += 3 * n * sizeof(double);
+  return PCG_OK;
+}
 // check_overflow at the end of complete steps, the stream idle
 int check_step_overflow(DeviceBatch &B) {
   volatile int *flag = B.d.ovf;
@@ -1368,13 +1378,11 @@ void enqueue_step(DeviceBatch &B) {
   const DevBatch &d = B.d;
   const pcg_params &p = B.hp.p;
   if (B.box_set) launch_box_phase(d, B.dP, sys_rw(B), B.stream);
-  launch_step_begin(d, B.prec, p.qa_on, B.stream);
-  launch_fix_nl(d, B.max_n, B.max_nlcap, B.cell_words, B.stream, false);
-  launch_terms(d, B.prec, B.max_items, -1, 0, -1, B.stream);
+  launch_fix_nl(d, B.max_n, B.cell_words, B.stream, true, p.qa_on);
+  launch_step_terms(d, B.prec, B.max_n, true, B.stream);
   if (p.qa_on) launch_qa_finish(d, B.max_n, B.stream);
   if (B.hp.ljw_terms) launch_ljw_process(d, B.stream);
-  if (B.box_set) launch_box_log(d, B.stream);
-  launch_lang(d, B.prec, B.noise, B.stream, true);
+  launch_lang(d, B.prec, B.noise, B.stream, true, B.box_set);
 }
 
 // the host copy of the system descriptor after the box protocol moved the
@@ -1455,6 +1463,7 @@ int pcg_create(const pcg_params *p, const pcg_model *m, const pcg_options *o, pc
   if (rc) return rc;
   c->B->noise = opt.noise;
   if ((rc = watch_overflow(*c->B))) return rc;
+  if ((rc = stage_forces(*c->B))) return rc;
   {
     DeviceBatch &B = *c->B;
     c->pcfg = persistent_cfg(B);
@@ -1551,7 +1560,7 @@ int pcg_fix_nl(pcg_ctx *c) {
   int rc = switch_form(*c, FORM_STAGES);
   if (rc) return rc;
   launch_mark_invalid(B.d, B.stream);
-  launch_fix_nl(B.d, B.max_n, B.max_nlcap, B.cell_words, B.stream);
+  launch_fix_nl(B.d, B.max_n, B.cell_words, B.stream, false, 0);
   return check_overflow(B);
 }
 
@@ -1570,8 +1579,9 @@ int pcg_eval_forces(pcg_ctx *c) {
   HIPCHK(hipSetDevice(B.device));
   int rc = switch_form(*c, FORM_STAGES);
   if (rc) return rc;
-  launch_eval_begin(B.d, B.prec, B.stream);
-  launch_terms(B.d, B.prec, B.max_items, -1, 0, -1, B.stream);
+  launch_eval_begin(B.d, B.stream);
+  launch_step_terms(B.d, B.prec, B.max_n, false, B.stream);
+  if (B.prec != PCG_FP64) launch_store_forces(B.d, B.stream);
   launch_tick(B.d, 0, B.stream);
   return check_overflow(B);
 }
@@ -1623,10 +1633,12 @@ static int eval_term_only(pcg_ctx *c, int32_t term, int32_t from, int32_t to, bo
   HIPCHK(hipSetDevice(B.device));
   const size_t at = (sizeof(SysState) + 255) / 256 * 256;
   if ((rc = B.pin->room(at + (want_F ? 24 * (size_t)B.sys[0].n : 0)))) return rc;
-  launch_eval_begin(B.d, B.prec, B.stream);
+  launch_eval_begin(B.d, B.stream);
   launch_terms(B.d, B.prec, B.max_items, term, from, to, B.stream);
   Fetch f;
   if (want_F) f = fetch_of(B, 0, B.d.F, B.prec != PCG_FP64, at);
+  if (want_F) f.acc = B.acc;
+  else if (B.acc) launch_store_forces(B.d, B.stream);
   f.src = B.d.st;
   f.dst = B.pin->p;
   f.bytes = sizeof(SysState);
@@ -1680,6 +1692,9 @@ int pcg_lang_step(pcg_ctx *c) {
   int rc = switch_form(*c, FORM_STAGES);
   if (rc) return rc;
   if (B.noise == PCG_NOISE_RAN2 && (rc = upload_ran2_noise(B))) return rc;
+  // the forces it takes are those a caller sees: an evaluation's, a step's or
+  // a restored state's
+  if (B.prec != PCG_FP64) launch_load_forces(B.d, B.stream);
   launch_lang(B.d, B.prec, B.noise, B.stream);
   launch_tick(B.d, 1, B.stream);
   HIPCHK(hipStreamSynchronize(B.stream));
@@ -2028,6 +2043,7 @@ int pcg_batch_create(const pcg_params *p, int32_t nsys, const pcg_model *models,
   const PersistentCfg pc = persistent_cfg(B);
   b->lds = pc.lds;
   b->persistent = pc.ok;
+  if (!pc.ok && (rc = stage_forces(B))) return rc;
   b->lean = pc.lean;
   if (opt.block != 0 && (opt.block < 64 || opt.block > 1024 || opt.block % 64 != 0))
     return fail(PCG_E_ARG, "block must be a multiple of 64 in [64, 1024]");

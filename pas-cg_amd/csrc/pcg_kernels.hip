@@ -12,29 +12,36 @@
 namespace pcg {
 
 // ------------------------------------------------------------ begin step ----
-// st.V zeroed; NL verify decision (nl::verify, cg/src/cg/nl/verify.cpp:3-34)
-// from the displacement maximum the previous Langevin step left behind.
-__device__ __forceinline__ void begin_system(const DevBatch &b, int s) {
+// NL verify decision (nl::verify, cg/src/cg/nl/verify.cpp:3-34) from the
+// displacement maximum the previous Langevin step left behind. Read only: in a
+// step, every thread of the first kernel takes it, and a later kernel
+// (k_step_terms) resets the scalars it reads.
+__device__ __forceinline__ bool rebuild_due(const DevBatch &b, int s) {
 #pragma clang fp contract(off)
-  SysState &st = b.st[s];
+  const SysState &st = b.st[s];
+  if (!b.P->nl_required) return st.nl_invalid != 0;
+  if (st.verify_first) return true;
   SysDescC &d = b.sys[s];
-  if (!st.active) return;
-  for (int k = 0; k < NT; ++k) st.V[k] = 0.0;
-  if (b.wall)  // dynamics::reset (dynamics.cpp:11-19) of the wall forces
+  const double maxd = __longlong_as_double((long long)st.max_disp_bits);
+  const double box = fabs(d.cell[0] - st.orig_cell[0]) + fabs(d.cell[1] - st.orig_cell[1]) +
+                     fabs(d.cell[2] - st.orig_cell[2]);
+  return __dadd_rn(__dmul_rn(2.0, maxd), box) > st.orig_pad;
+}
+// a system's energies and the walls' reaction forces at zero
+// (dynamics::reset, dynamics.cpp:11-19)
+__device__ __forceinline__ void clear_system(const DevBatch &b, int s) {
+  for (int k = 0; k < NT; ++k) b.st[s].V[k] = 0.0;
+  if (b.wall)
     for (int w = 0; w < 6; ++w)
       for (int c = 0; c < 3; ++c) b.wall->wall_F[w][c] = 0.0;
-  if (b.P->nl_required) {
-    if (st.verify_first) {
-      st.verify_first = 0;
-      st.nl_invalid = 1;
-    } else {
-      double maxd = __longlong_as_double((long long)st.max_disp_bits);
-      double box = fabs(d.cell[0] - st.orig_cell[0]) + fabs(d.cell[1] - st.orig_cell[1]) +
-                   fabs(d.cell[2] - st.orig_cell[2]);
-      double disp = __dadd_rn(__dmul_rn(2.0, maxd), box);
-      st.nl_invalid = disp > st.orig_pad ? 1 : 0;
-    }
-  }
+}
+// the verify outside a step
+__device__ __forceinline__ void begin_system(const DevBatch &b, int s) {
+  SysState &st = b.st[s];
+  if (!st.active) return;
+  clear_system(b, s);
+  st.nl_invalid = rebuild_due(b, s) ? 1 : 0;
+  if (b.P->nl_required) st.verify_first = 0;
   st.max_disp_bits = 0ull;
 }
 
@@ -44,20 +51,42 @@ __global__ void k_begin(DevBatch b) {
   begin_system(b, s);
 }
 
-// Before an evaluation outside a step: forces, energies and the walls'
-// reaction forces at zero.
-template <typename RF> __global__ void k_eval_begin(DevBatch b) {
+// Residue i before an evaluation: its force at zero; the system's first one
+// clears the rest.
+__device__ __forceinline__ void clear_residue(const DevBatch &b, int i, int s) {
+  if (b.local[i] == 0) clear_system(b, s);
+  for (int c = 0; c < 3; ++c) b.acc[c][i] = 0.0;
+}
+// an evaluation outside a step
+__global__ void k_eval_begin(DevBatch b) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= b.ntot) return;
   const int s = b.sysid[i];
-  if (b.local[i] == 0) {
-    for (int k = 0; k < NT; ++k) b.st[s].V[k] = 0.0;
-    if (b.wall)
-      for (int w = 0; w < 6; ++w)
-        for (int c = 0; c < 3; ++c) b.wall->wall_F[w][c] = 0.0;
-  }
   if (!b.st[s].active) return;
-  for (int c = 0; c < 3; ++c) ((RF *)b.F[c])[i] = 0;
+  clear_residue(b, i, s);
+}
+// Residue i at the start of a step: cleared, its n and h (qa_on); the
+// system's first residue writes down whether the step rebuilds its lists
+// (due), for the kernels after this one.
+__device__ __forceinline__ void begin_residue(const DevBatch &b, int i, int s, bool due, int qa_on) {
+  if (!b.st[s].active) return;
+  clear_residue(b, i, s);
+  if (b.local[i] == 0) b.st[s].nl_invalid = due ? 1 : 0;
+  if (qa_on) {
+    GeoG g{b.y[0][0], b.y[0][1], b.y[0][2]};
+    prepare_nh_item(b, g, i);
+  }
+}
+// the forces of an evaluation, accumulated in FP64, into the FP32 arrays
+// (STORE), or back for an integration outside a step
+template <bool STORE> __global__ void k_move_forces(DevBatch b) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= b.ntot) return;
+  for (int c = 0; c < 3; ++c) {
+    float *f = (float *)b.F[c];
+    if (STORE) f[i] = (float)b.acc[c][i];
+    else b.acc[c][i] = f[i];
+  }
 }
 
 // The next rebuild of every system is due.
@@ -75,12 +104,15 @@ __global__ void k_mark_invalid(DevBatch b) {
 // 14 us with a wait for the stream, 47 us as three staged column copies).
 template <typename T>
 __global__ __launch_bounds__(1024) void k_fetch(const uint32_t *words, uint32_t *words_out, int nw,
-                                                const T *x, const T *y, const T *z, double *out,
-                                                int n, int *flag, int seq) {
+                                                const T *x, const T *y, const T *z,
+                                                const double *acc, double *out, int n, int *flag,
+                                                int seq) {
   for (int i = threadIdx.x; i < nw; i += blockDim.x) words_out[i] = words[i];
   for (int i = threadIdx.x; i < 3 * n; i += blockDim.x) {
     const int k = i / 3, c = i - 3 * k;
-    out[i] = (double)(c == 0 ? x : c == 1 ? y : z)[k];
+    const T *col = c == 0 ? x : c == 1 ? y : z;
+    if (acc) ((T *)col)[k] = (T)acc[(size_t)c * n + k];
+    out[i] = (double)col[k];
   }
   if (!flag) return;
   // every wave's stores are out before the barrier; one release covers them
@@ -112,18 +144,19 @@ __device__ __forceinline__ bool nl_pred(const DevBatch &b, SysDescC &s, const Ge
 }
 
 // Completion count of a per-item stage kernel: every lane with `mine` (an
-// item of system `sys`) counts itself toward the system's residue count in
-// the SysState field `done`; a wave whose counted lanes share one system
+// item of system `sys`) counts itself toward the system's residue count
+// (and extra more items) in the SysState field `done`; a wave whose counted lanes share one system
 // adds them with one atomic. Returns, in the lane whose add completed a
-// system, that system (-1 elsewhere); what every lane wrote before the call
-// is visible to it then.
+// system, that system (-1 elsewhere); with fence, what every lane wrote before
+// the call is visible to it then.
 __device__ __forceinline__ int count_done(const DevBatch &b, int SysState::*done, bool mine,
-                                          int sys) {
+                                          int sys, bool fence = true, int extra = 0) {
   // a wave with nothing to count skips the fence: an agent-scope release
   // writes back the L2, and on a step without a rebuild every wave of the
   // cell count has nothing to count
   if (!__any(mine)) return -1;
-  __threadfence();
+  if (fence) __threadfence();
+  else __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // what was read, was read
   const int lane = threadIdx.x & 63;
   const unsigned long long m = __ballot(mine);
   const int sys0 = __shfl(sys, 0, 64);
@@ -136,8 +169,8 @@ __device__ __forceinline__ int count_done(const DevBatch &b, int SysState::*done
   }
   if (who < 0) return -1;
   const int old = atomicAdd(&(b.st[who].*done), add);
-  if (old + add != b.sys[who].n) return -1;
-  __threadfence();
+  if (old + add != b.sys[who].n + extra) return -1;
+  if (fence) __threadfence();
   return who;
 }
 
@@ -158,35 +191,38 @@ __device__ __forceinline__ int wave_incl(int x, int &total) {
   return x;
 }
 
-// One wave's exclusive scan of v[0..n) in place, also into also[0..n) when
-// given; returns the total in every lane. The wave walks v in stripes of 64
-// consecutive entries, loading 16 stripes at once (coalesced, all in flight
-// together) and carrying the running sum from stripe to stripe. Every lane
-// of the wave must be active.
-__device__ __forceinline__ int wave_scan(int *v, int n, int *also) {
-  constexpr int SB = 16;
+// One wave's exclusive scans of M arrays v[m][0..n) in place, the first one
+// also into also[0..n) when given; their totals in every lane. The wave walks
+// the arrays in stripes of 64 consecutive entries, loading SB stripes of each
+// at once (coalesced, all in flight together) and carrying the running sums
+// from stripe to stripe. Every lane of the wave must be active.
+template <int M, int SB>
+__device__ __forceinline__ void wave_scan(int *const (&v)[M], int n, int *also, int (&total)[M]) {
   const int lane = threadIdx.x & 63;
-  int carry = 0;
+  for (int m = 0; m < M; ++m) total[m] = 0;
   for (int base = 0; base < n; base += 64 * SB) {
-    int x[SB];
+    int x[M][SB];
 #pragma unroll
-    for (int j = 0; j < SB; ++j) {
-      const int k = base + j * 64 + lane;
-      x[j] = k < n ? v[k] : 0;
-    }
+    for (int m = 0; m < M; ++m)
 #pragma unroll
-    for (int j = 0; j < SB; ++j) {
-      int tot;
-      const int inc = wave_incl(x[j], tot);
-      const int k = base + j * 64 + lane;
-      if (k < n) {
-        v[k] = carry + inc - x[j];
-        if (also) also[k] = carry + inc - x[j];
+      for (int j = 0; j < SB; ++j) {
+        const int k = base + j * 64 + lane;
+        x[m][j] = k < n ? v[m][k] : 0;
       }
-      carry += tot;
-    }
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+      for (int j = 0; j < SB; ++j) {
+        int tot;
+        const int inc = wave_incl(x[m][j], tot);
+        const int k = base + j * 64 + lane;
+        if (k < n) {
+          v[m][k] = total[m] + inc - x[m][j];
+          if (m == 0 && also) also[k] = total[m] + inc - x[m][j];
+        }
+        total[m] += tot;
+      }
   }
-  return carry;
 }
 
 // ------------------------------------------------------------- cell grid ----
@@ -213,10 +249,11 @@ __device__ __forceinline__ int cell_coord(SysDescC &sd, int a, double x) {
   return k < 0 ? 0 : (k >= sd.cg[a] ? sd.cg[a] - 1 : k);
 }
 
-// each residue's cell; cell_end counts the residues of each cell; the wave
+// A step's first kernel when a system is on a cell grid (begin): the residues'
+// begin work. Each residue's cell; cell_end counts the residues of each cell; the wave
 // whose residue completes a system turns its counts into the cells' first
 // slots (cell_start) and fill pointers (cell_end)
-__global__ void k_cell_count(DevBatch b) {
+__global__ void k_cell_count(DevBatch b, int begin, int qa_on) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   bool mine = false;
   int sys = -1;
@@ -224,7 +261,9 @@ __global__ void k_cell_count(DevBatch b) {
     sys = b.sysid[i];
     const SysState &st = b.st[sys];
     SysDescC &sd = b.sys[sys];
-    if (st.active && st.nl_invalid && use_cells(b, sd)) {
+    const bool due = begin ? rebuild_due(b, sys) : st.nl_invalid != 0;
+    if (begin) begin_residue(b, i, sys, due, qa_on);
+    if (st.active && due && use_cells(b, sd)) {
       mine = true;
       const int c = (cell_coord(sd, 2, b.y[0][2][i]) * sd.cg[1] + cell_coord(sd, 1, b.y[0][1][i])) *
                         sd.cg[0] + cell_coord(sd, 0, b.y[0][0][i]);
@@ -239,9 +278,17 @@ __global__ void k_cell_count(DevBatch b) {
     dm &= dm - 1ull;
     const int ds = __shfl(done, src, 64);
     SysDescC &sd = b.sys[ds];
-    wave_scan(b.cell_end + sd.cell0, sd.cg[0] * sd.cg[1] * sd.cg[2], b.cell_start + sd.cell0);
+    int *const v[1] = {b.cell_end + sd.cell0};
+    int total[1];
+    wave_scan<1, 16>(v, sd.cg[0] * sd.cg[1] * sd.cg[2], b.cell_start + sd.cell0, total);
     if ((threadIdx.x & 63) == 0) b.st[ds].done_cells = 0;
   }
+}
+
+// the cell counts back to zero for the next rebuild, once the rows are written
+__device__ __forceinline__ void clear_cells(const DevBatch &b, SysDescC &sd, int t, int nt) {
+  const int nc = sd.cg[0] > 0 ? sd.cg[0] * sd.cg[1] * sd.cg[2] : 0;
+  for (int c = t; c < nc; c += nt) b.cell_end[sd.cell0 + c] = 0;
 }
 
 // the residues into their cells' slots (any order within a cell: a row's
@@ -258,43 +305,187 @@ __global__ void k_cell_fill(DevBatch b) {
   b.cell_items[sd.res0 + slot] = i - sd.res0;
 }
 
-// cell_words: 64-bit mask words of the largest system on the grid (the
-// dynamic LDS holds one row mask a wave), 0 without a grid
-// The rows' counts of system s into their first slots, by one whole wave;
-// then the list's length and the rebuild's snapshot of the pad and cell.
-__device__ __forceinline__ void nl_scan_tail(const DevBatch &b, int s) {
-  SysState &st = b.st[s];
-  SysDescC &sd = b.sys[s];
-  const int tot = wave_scan(b.row_cnt + sd.res0, sd.n, nullptr);
-  if ((threadIdx.x & 63) == 0) {
-    st.nl_n = tot > sd.nlcap ? sd.nlcap : tot;
+// Per-row counts of a rebuild: the NL pairs in row_cnt, the lists the pairs go
+// to (RC_*) in the system's candidate scratch, which only a step's QA stage
+// uses; [class][residue within the system]. After the scan, the rows' first
+// slots.
+enum { RC_NC, RC_QA, RC_NEAR, RC_PID, RC_DH, RC_PAULI, RC_N };
+__device__ __forceinline__ int *row_counts(const DevBatch &b, SysDescC &sd, int cls) {
+  return b.cand_perm + sd.nl0 + cls * sd.n;
+}
+
+__device__ __forceinline__ int *nl_counts(const DevBatch &b, SysDescC &sd) {
+  return b.row_cnt + sd.res0;
+}
+
+// the length of the NL (cls -1) or of one of the lists
+__device__ __forceinline__ void set_length(SysState &st, SysDescC &sd, int cls, int tot) {
+  const int qf = min(tot, sd.qfcap), nl = min(tot, sd.nlcap);
+  switch (cls) {
+  case -1:
+    st.nl_n = nl;
     if (tot > sd.nlcap) st.overflow = 1;
-    // the list updates filter with the new pad (legacy_update.cpp:84)
-    st.orig_pad = b.P->p.nl_pad;
-    for (int c = 0; c < 3; ++c) st.orig_cell[c] = sd.cell[c];
+    break;
+  case RC_NC: st.nc_n = tot; break;
+  case RC_QA:
+    st.qf_n = qf;
+    st.qf_store = qf;
+    if (tot > sd.qfcap) st.overflow = 1;
+    break;
+  case RC_NEAR: st.qh_n = qf; break;
+  case RC_PID: st.pid_n = nl; break;
+  case RC_DH: st.dh_n = nl; break;
+  case RC_PAULI: st.pauli_n = nl; break;
   }
 }
 
-template <bool WRITE> __global__ void k_nl_rows(DevBatch b, int cell_words, int fuse_scan) {
+// One row of the sorted NL by one wave, with the ordered list updates of
+// thread::fix_nl_async (thread_main.cpp:409-423): native contacts take first
+// (nat_cont/update_contacts.cpp:7-37), then QA free pairs
+// (qa/update_free_pairs.cpp:4-25), PID bundles and DH pairs see the rest
+// without taking (pid/update_bundles.cpp:4-34, dh/update_pairs.cpp:4-25),
+// Pauli takes last (pauli/update_pairs.cpp:4-20). Each pair's destination
+// depends only on the pair, so the first pass counts each list's pairs per row
+// (WRITE false), a scan gives every row its slots, and the second pass writes
+// the NL pair and its list entries there. (Classifying in the rows instead of
+// over the finished NL saves two launches, 5.7 us of a step with or without a
+// rebuild, and the NL's reading back.)
+template <bool WRITE> struct RowOut {
+  const DevBatch &b;
+  SysDescC &sd;
+  int row, il, out, at[RC_N];
+  int c0, nc;     // the row's native contacts [c0, c0 + nc) of all
+  int partner;    // their second residues, one a lane (of the first 64)
+  __device__ __forceinline__ RowOut(const DevBatch &b_, SysDescC &sd_, int row_)
+      : b(b_), sd(sd_), row(row_), il(row_ - sd_.res0) {
+    const int lane = threadIdx.x & 63;
+    out = WRITE ? b.row_cnt[row] : 0;
+    for (int c = 0; c < RC_N; ++c) at[c] = WRITE ? row_counts(b, sd, c)[il] : 0;
+    // contacts are sorted by (i1, i2): the first of this row by bisection
+    int lo = sd.nc0, hi = sd.nc0 + (b.P->p.nat_cont_on ? sd.nnc : 0);
+    const int end = hi;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (b.nc_i[0][mid] < row) lo = mid + 1;
+      else hi = mid;
+    }
+    c0 = __builtin_amdgcn_readfirstlane(lo);
+    const bool mine = c0 + lane < end && b.nc_i[0][c0 + lane] == row;
+    partner = mine ? b.nc_i[1][c0 + lane] : -1;
+    nc = __popcll(__ballot(mine));
+  }
+  // the contact of residue j in this row, or -1
+  __device__ __forceinline__ int contact(int j) const {
+    int found = -1;
+    for (int m = nc - 1; m >= 0; --m)
+      if (__builtin_amdgcn_readlane(partner, m) == j) found = c0 + m;
+    if (nc == 64 && found < 0) found = find_contact(b, sd, row, j);  // more than 64 contacts
+    return found;
+  }
+  // 64 pairs (row, j), of which the lanes with `in` are NL pairs at distance d
+  __device__ __forceinline__ void pairs(int j, bool in, double d) {
+    const unsigned long long m = __ballot(in);
+    if (!m) return;
+    const int nat = contact(j);
+    const int cls = in ? classify(b, sd, row, j, d, nat >= 0) : 0;
+    const unsigned long long mm[RC_N] = {
+        __ballot(cls & CL_NC), __ballot(cls & CL_QA), __ballot(cls & CL_NEAR),
+        __ballot(cls & CL_PID), __ballot(cls & CL_DH), __ballot(cls & CL_PAULI)};
+    if (WRITE && in) {
+      const unsigned long long below = (1ull << (threadIdx.x & 63)) - 1ull;
+      auto slot = [&](int c) { return at[c] + __popcll(mm[c] & below); };
+      const int pos = out + __popcll(m & below);
+      if (pos < sd.nlcap) {
+        b.nl_i[0][sd.nl0 + pos] = row;
+        b.nl_i[1][sd.nl0 + pos] = j;
+        b.nl_d[sd.nl0 + pos] = d;
+      }
+      if (cls & CL_NC) set_current_contact(b, sd.nc0 + slot(RC_NC), nat, sd.res0);
+      if (cls & CL_QA) {
+        const int p = slot(RC_QA), q = sd.qf0 + p;
+        if (p < sd.qfcap) {
+          b.qf_i[0][q] = row;
+          b.qf_i[1][q] = j;
+          b.qf_d[q] = d;
+          b.qf_vac[q] = 0;
+          if (cls & CL_NEAR) {
+            // near list entry: the free pair in slot p (its order is the
+            // free pairs' order)
+            const int h = sd.qf0 + slot(RC_NEAR);
+            b.qh_slot[h] = p;
+            b.qh_i[0][h] = row;
+            b.qh_i[1][h] = j;
+            b.qh_vac[h] = 0;
+            qa_near_filters(b, row, j, b.qh_req[h], b.qh_thr2[h]);
+            b.qh_ij[h] = (uint32_t)il | ((uint32_t)(j - sd.res0) << 16);
+          }
+        }
+      }
+      if (cls & CL_PID) {
+        const int p = slot(RC_PID), q = sd.nl0 + p;
+        if (p < sd.nlcap) {
+          b.pid_i[0][q] = row;
+          b.pid_i[1][q] = j;
+          b.pid_d[q] = d;
+          b.pid_t[q] = (int16_t)(b.atype[row] * 21 + b.atype[j]);
+        }
+      }
+      if (cls & CL_DH) {
+        const int p = slot(RC_DH), q = sd.nl0 + p;
+        if (p < sd.nlcap) {
+          b.dh_i[0][q] = row;
+          b.dh_i[1][q] = j;
+          b.dh_q[q] = b.P->p.charge[b.atype[row]] * b.P->p.charge[b.atype[j]];
+        }
+      }
+      if (cls & CL_PAULI) {
+        const int p = slot(RC_PAULI), q = sd.nl0 + p;
+        if (p < sd.nlcap) {
+          b.pauli_i[0][q] = row;
+          b.pauli_i[1][q] = j;
+        }
+      }
+    }
+    out += __popcll(m);
+    for (int c = 0; c < RC_N; ++c) at[c] += __popcll(mm[c]);
+  }
+};
+
+// cell_words: 64-bit mask words of the largest system on the grid (the
+// dynamic LDS holds one row mask a wave), 0 without a grid. begin (the count
+// pass, without a grid): the step's first kernel, whose first threads do the
+// residues' begin work.
+template <bool WRITE>
+__global__ void k_nl_rows(DevBatch b, int cell_words, int fuse_scan, int begin, int qa_on) {
   extern __shared__ unsigned long long row_mask[];
-  int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  int lane = threadIdx.x & 63;
+  if (!WRITE && begin) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < b.ntot) begin_residue(b, i, b.sysid[i], rebuild_due(b, b.sysid[i]), qa_on);
+  }
+  const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
   if (row >= b.ntot) return;
-  int s = b.sysid[row];
+  const int s = b.sysid[row];
   SysState &st = b.st[s];
-  if (!st.active || !st.nl_invalid) return;
+  if (!st.active || !(!WRITE && begin ? rebuild_due(b, s) : st.nl_invalid != 0)) return;
   SysDescC &sd = b.sys[s];
   GeoG g{b.y[0][0], b.y[0][1], b.y[0][2]};
-  // the snapshot of the rebuild's positions (legacy_update.cpp:80-89)
-  if (WRITE && lane == 0)
+  // the snapshot of the rebuild's positions, pad and cell
+  // (legacy_update.cpp:80-89); in the second pass, as a step's verify, taken
+  // by the threads of the first, reads the old one
+  if (WRITE && lane == 0) {
     for (int c = 0; c < 3; ++c) b.orig_r[c][row] = b.y[0][c][row];
-  double req = b.P->nl_eff_cutoff + b.P->p.nl_pad;
-  int end = sd.res0 + sd.n;
-  int out = WRITE ? b.row_cnt[row] : 0;
-  int cnt = 0;
+    if (row == sd.res0) {
+      st.orig_pad = b.P->p.nl_pad;
+      for (int c = 0; c < 3; ++c) st.orig_cell[c] = sd.cell[c];
+    }
+  }
+  const double req = b.P->nl_eff_cutoff + b.P->p.nl_pad;
+  const int end = sd.res0 + sd.n;
+  RowOut<WRITE> o(b, sd, row);
   if (cell_words > 0 && use_cells(b, sd)) {
     unsigned long long *m = row_mask + (size_t)(threadIdx.x >> 6) * cell_words;
-    const int il = row - sd.res0, W = (sd.n + 63) >> 6, w0 = (il + 1) >> 6;
+    const int il = o.il, W = (sd.n + 63) >> 6, w0 = (il + 1) >> 6;
     for (int w = w0 + lane; w < W; w += 64) m[w] = 0ull;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -305,9 +496,9 @@ template <bool WRITE> __global__ void k_nl_rows(DevBatch b, int cell_words, int 
       for (int dy = -1; dy <= 1; ++dy)
         for (int dx = -1; dx <= 1; ++dx) {
           const int nx = (cx + dx + gx) % gx, ny = (cy + dy + gy) % gy, nz = (cz + dz + gz) % gz;
-          const int nc = sd.cell0 + (nz * gy + ny) * gx + nx;
-          const int t1 = b.cell_end[nc];
-          for (int t = b.cell_start[nc] + lane; t < t1; t += 64) {
+          const int ncell = sd.cell0 + (nz * gy + ny) * gx + nx;
+          const int t1 = b.cell_end[ncell];
+          for (int t = b.cell_start[ncell] + lane; t < t1; t += 64) {
             const int j = b.cell_items[sd.res0 + t];
             if (j > il) atomicOr(&m[j >> 6], 1ull << (j & 63));
           }
@@ -326,42 +517,25 @@ template <bool WRITE> __global__ void k_nl_rows(DevBatch b, int cell_words, int 
         const unsigned long long bw = (unsigned long long)lo | ((unsigned long long)hi << 32);
         const int j = sd.res0 + (wb + k) * 64 + lane;
         double dist = 0.0;
-        const bool keep = ((bw >> lane) & 1ull) && nl_pred(b, sd, g, row, j, req, dist);
-        const unsigned long long mm = __ballot(keep);
-        if (WRITE && keep) {
-          int pos = out + cnt + __popcll(mm & ((1ull << lane) - 1ull));
-          if (pos < sd.nlcap) {
-            int slot = sd.nl0 + pos;
-            b.nl_i[0][slot] = row;
-            b.nl_i[1][slot] = j;
-            b.nl_d[slot] = dist;
-          }
-        }
-        cnt += __popcll(mm);
+        const bool in = ((bw >> lane) & 1ull) && nl_pred(b, sd, g, row, j, req, dist);
+        o.pairs(j, in, dist);
       }
     }
   } else {
-  for (int j0 = row + 1; j0 < end; j0 += 64) {
-    int j = j0 + lane;
-    double dist = 0.0;
-    bool keep = j < end && nl_pred(b, sd, g, row, j, req, dist);
-    unsigned long long m = __ballot(keep);
-    if (WRITE && keep) {
-      int pos = out + cnt + __popcll(m & ((1ull << lane) - 1ull));
-      if (pos < sd.nlcap) {
-        int slot = sd.nl0 + pos;
-        b.nl_i[0][slot] = row;
-        b.nl_i[1][slot] = j;
-        b.nl_d[slot] = dist;
-      }
+    for (int j0 = row + 1; j0 < end; j0 += 64) {
+      const int j = j0 + lane;
+      double dist = 0.0;
+      const bool in = j < end && nl_pred(b, sd, g, row, j, req, dist);
+      o.pairs(j, in, dist);
     }
-    cnt += __popcll(m);
-  }
   }
   if (!WRITE) {
     // the row counts; with fuse_scan the wave of the system's last row to
     // finish scans them into the rows' first slots, else k_nl_scan does
-    if (lane == 0) b.row_cnt[row] = cnt;
+    if (lane == 0) {
+      b.row_cnt[row] = o.out;
+      for (int c = 0; c < RC_N; ++c) row_counts(b, sd, c)[o.il] = o.at[c];
+    }
     if (!fuse_scan) return;
     int fin = 0;
     if (lane == 0) {
@@ -370,14 +544,22 @@ template <bool WRITE> __global__ void k_nl_rows(DevBatch b, int cell_words, int 
     }
     if (__shfl(fin, 0, 64)) {
       __threadfence();
-      nl_scan_tail(b, s);
-      if (lane == 0) st.done_rows = 0;
+      int *const v[RC_N + 1] = {nl_counts(b, sd),         row_counts(b, sd, 0),
+                                row_counts(b, sd, 1), row_counts(b, sd, 2),
+                                row_counts(b, sd, 3), row_counts(b, sd, 4),
+                                row_counts(b, sd, 5)};
+      int total[RC_N + 1];
+      wave_scan<RC_N + 1, 4>(v, sd.n, nullptr, total);
+      if (lane == 0) {
+        for (int c = -1; c < RC_N; ++c) set_length(st, sd, c, total[c + 1]);
+        st.done_rows = 0;
+      }
     }
   }
 }
 
-// The row scan as a launch of its own, one wave a system: for systems of
-// ROWS_FUSE_MAX residues or more. Every row's count comes to its system's
+// The row scan as a launch of its own, one wave a system and list: for systems
+// of ROWS_FUSE_MAX residues or more. Every row's count comes to its system's
 // counter through an agent-scope fence, and on this device such a fence
 // writes back and invalidates the L2: in the trace of a 6400-residue box a
 // rebuild's count pass took 131 us with the fused scan and about 20 us
@@ -385,228 +567,38 @@ template <bool WRITE> __global__ void k_nl_rows(DevBatch b, int cell_words, int 
 __global__ void k_nl_scan(DevBatch b) {
   const int s = blockIdx.x;
   if (s >= b.nsys) return;
-  const SysState &st = b.st[s];
-  if (!st.active || !st.nl_invalid) return;
-  nl_scan_tail(b, s);
-}
-
-// ------------------------------------------------------------ list updates ----
-// The ordered updates of thread::fix_nl_async (thread_main.cpp:409-423):
-// native contacts take first (nat_cont/update_contacts.cpp:7-37), then QA
-// free pairs (qa/update_free_pairs.cpp:4-25), PID bundles and DH pairs see the
-// rest without taking (pid/update_bundles.cpp:4-34, dh/update_pairs.cpp:4-25),
-// Pauli takes last (pauli/update_pairs.cpp:4-20). Each NL pair's destination
-// depends only on the pair, so the partition is one classification pass plus
-// an order-preserving compaction per list.
-__device__ __forceinline__ void block_counts6(int cls, int valid, int counts[NCL], int ranks[NCL]) {
-  // ordered rank of this thread within the block for each class, and totals
-  __shared__ int wc[BLK / 64][NCL];
-  int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  unsigned long long lt = (1ull << lane) - 1ull;
-  int mine[NCL];
-  for (int c = 0; c < NCL; ++c) {
-    unsigned long long m = __ballot(valid && (cls & (1 << c)));
-    mine[c] = __popcll(m & lt);
-    if (lane == 0) wc[w][c] = __popcll(m);
-  }
-  __syncthreads();
-  for (int c = 0; c < NCL; ++c) {
-    int off = 0, tot = 0;
-    for (int k = 0; k < nw; ++k) {
-      if (k < w) off += wc[k][c];
-      tot += wc[k][c];
-    }
-    ranks[c] = off + mine[c];
-    counts[c] = tot;
-  }
-  __syncthreads();
-}
-
-// One block of system s: every class's per-chunk counts become their exclusive
-// prefix in chunk order, and the totals the lists' sizes. Each thread takes
-// a contiguous run of chunks; a scan over the threads gives each run its
-// offsets.
-__device__ __forceinline__ void part_scan_block(const DevBatch &b, int s) {
-  SysState &st = b.st[s];
-  SysDescC &sd = b.sys[s];
-  const int nchunks = (st.nl_n + BLK - 1) / BLK, T = blockDim.x;
-  const int per = (nchunks + T - 1) / T;
-  const int c0 = min((int)threadIdx.x * per, nchunks), c1 = min(c0 + per, nchunks);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = T >> 6;
-  __shared__ int wsum[BLK / 64][NCL];
-  int run[NCL], tot[NCL];
-  for (int c = 0; c < NCL; ++c) run[c] = 0;
-  for (int ch = c0; ch < c1; ++ch)
-    for (int c = 0; c < NCL; ++c) run[c] += b.blk_cnt[(sd.nl0 / BLK + ch) * NCL + c];
-  for (int c = 0; c < NCL; ++c) {
-    int x = run[c];
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(x, o, 64);
-      if (lane >= o) x += y;
-    }
-    if (lane == 63) wsum[w][c] = x;
-    run[c] = x - run[c];  // exclusive within the wave
-  }
-  __syncthreads();
-  for (int c = 0; c < NCL; ++c) {
-    int off = 0, t = 0;
-    for (int k = 0; k < nw; ++k) {
-      if (k < w) off += wsum[k][c];
-      t += wsum[k][c];
-    }
-    run[c] += off;
-    tot[c] = t;
-  }
-  for (int ch = c0; ch < c1; ++ch)
-    for (int c = 0; c < NCL; ++c) {
-      const int at = (sd.nl0 / BLK + ch) * NCL + c, v = b.blk_cnt[at];
-      b.blk_cnt[at] = run[c];
-      run[c] += v;
-    }
-  if (threadIdx.x == 0) {
-    st.nc_n = tot[0];
-    st.qf_n = tot[1] < sd.qfcap ? tot[1] : sd.qfcap;
-    st.qf_store = st.qf_n;
-    if (tot[1] > sd.qfcap) st.overflow = 1;
-    st.pid_n = tot[2];
-    st.dh_n = tot[3];
-    st.pauli_n = tot[4];
-    st.qh_n = tot[5] < sd.qfcap ? tot[5] : sd.qfcap;
-  }
-}
-
-// One chunk of BLK pairs of system s: each pair's classes, and the chunk's
-// count per class
-__device__ __forceinline__ void part_count_chunk(DevBatch &b, SysDescC &sd, const SysState &st,
-                                                 int ch) {
-  int k = ch * BLK + (int)threadIdx.x;
-  int valid = k < st.nl_n;
-  int cls = valid ? classify(b, sd, st, sd.nl0 + k) : 0;
-  if (valid) b.nl_cls[sd.nl0 + k] = (uint8_t)cls;
-  int counts[NCL], ranks[NCL];
-  block_counts6(cls, valid, counts, ranks);
-  if (threadIdx.x == 0) {
-    int base = (sd.nl0 / BLK + ch) * NCL;
-    for (int c = 0; c < NCL; ++c) b.blk_cnt[base + c] = counts[c];
-  }
-}
-
-// blockIdx.y: system; the blocks stride over the chunks the list fills, so
-// a step without a rebuild costs a small grid's launch
-__global__ void k_part_count(DevBatch b) {
-  int s = blockIdx.y;
   SysState &st = b.st[s];
   if (!st.active || !st.nl_invalid) return;
   SysDescC &sd = b.sys[s];
-  // only the blocks with chunks or cells to visit take part (and count
-  // themselves below)
-  const int nchunks = (st.nl_n + BLK - 1) / BLK;
-  const int nc = sd.cg[0] > 0 ? sd.cg[0] * sd.cg[1] * sd.cg[2] : 0;
-  const int nb = max(1, min((int)gridDim.x, max(nchunks, (nc + BLK - 1) / BLK)));
-  if ((int)blockIdx.x >= nb) return;
-  // the cell counts start the next rebuild at zero (the rows are written)
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nc; c += nb * blockDim.x)
-    b.cell_end[sd.cell0 + c] = 0;
-  for (int ch = blockIdx.x; ch < nchunks; ch += nb) part_count_chunk(b, sd, st, ch);
-  // the system's last block to finish scans the chunk counts
-  __shared__ int last;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __threadfence();
-    last = atomicAdd(&st.done_part, 1) == nb - 1;
-  }
-  __syncthreads();
-  if (!last) return;
-  __threadfence();
-  part_scan_block(b, s);
-  if (threadIdx.x == 0) st.done_part = 0;
+  const int cls = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) - 1);
+  int *const v[1] = {cls < 0 ? nl_counts(b, sd) : row_counts(b, sd, cls)};
+  int total[1];
+  wave_scan<1, 16>(v, sd.n, nullptr, total);
+  if ((threadIdx.x & 63) == 0) set_length(st, sd, cls, total[0]);
 }
 
-// One chunk's pairs into their lists at the chunk's offsets (the scan of
-// k_part_count)
-__device__ __forceinline__ void part_write_chunk(DevBatch &b, SysDescC &sd, const SysState &st,
-                                                 int ch) {
-  int k = ch * BLK + (int)threadIdx.x;
-  int valid = k < st.nl_n;
-  int slot = sd.nl0 + k;
-  int cls = valid ? b.nl_cls[slot] : 0;
-  int counts[NCL], ranks[NCL];
-  block_counts6(cls, valid, counts, ranks);
-  if (!valid || !cls) return;
-  int base = (sd.nl0 / BLK + ch) * NCL;
-  int i1 = b.nl_i[0][slot], i2 = b.nl_i[1][slot];
-  double d = b.nl_d[slot];
-  ParamsC &p = b.P->p;
-  if (cls & CL_NC) {
-    int pos = b.blk_cnt[base + 0] + ranks[0];
-    set_current_contact(b, sd.nc0 + pos, find_contact(b, sd, i1, i2), sd.res0);
-  }
-  if (cls & CL_QA) {
-    int pos = b.blk_cnt[base + 1] + ranks[1];
-    if (pos < sd.qfcap) {
-      int q = sd.qf0 + pos;
-      b.qf_i[0][q] = i1;
-      b.qf_i[1][q] = i2;
-      b.qf_d[q] = d;
-      b.qf_vac[q] = 0;
-      if (cls & CL_NEAR) {
-        // near list entry: the free pair in slot pos (its order is the
-        // free pairs' order)
-        const int h = sd.qf0 + b.blk_cnt[base + 5] + ranks[5];
-        b.qh_slot[h] = pos;
-        b.qh_i[0][h] = i1;
-        b.qh_i[1][h] = i2;
-        b.qh_vac[h] = 0;
-        qa_near_filters(b, i1, i2, b.qh_req[h], b.qh_thr2[h]);
-        b.qh_ij[h] = (uint32_t)(i1 - sd.res0) | ((uint32_t)(i2 - sd.res0) << 16);
-      }
-    }
-  }
-  if (cls & CL_PID) {
-    int q = sd.nl0 + b.blk_cnt[base + 2] + ranks[2];
-    b.pid_i[0][q] = i1;
-    b.pid_i[1][q] = i2;
-    b.pid_d[q] = d;
-    b.pid_t[q] = (int16_t)(b.atype[i1] * 21 + b.atype[i2]);
-  }
-  if (cls & CL_DH) {
-    int q = sd.nl0 + b.blk_cnt[base + 3] + ranks[3];
-    b.dh_i[0][q] = i1;
-    b.dh_i[1][q] = i2;
-    b.dh_q[q] = p.charge[b.atype[i1]] * p.charge[b.atype[i2]];
-  }
-  if (cls & CL_PAULI) {
-    int q = sd.nl0 + b.blk_cnt[base + 4] + ranks[4];
-    b.pauli_i[0][q] = i1;
-    b.pauli_i[1][q] = i2;
-  }
-}
-
-
-__global__ void k_part_write(DevBatch b) {
-  int s = blockIdx.y;
-  const SysState &st = b.st[s];
-  if (!st.active || !st.nl_invalid) return;
-  SysDescC &sd = b.sys[s];
-  const int nchunks = (st.nl_n + BLK - 1) / BLK;
-  for (int ch = blockIdx.x; ch < nchunks; ch += gridDim.x) part_write_chunk(b, sd, st, ch);
-}
-
-// The rebuild is complete: record it and clear nl_invalid.
+// A rebuild outside a step is complete: record it and clear nl_invalid and the
+// cell counts; one block a system.
 __global__ void k_nl_done(DevBatch b) {
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= b.nsys) return;
+  const int s = blockIdx.x;
   SysState &st = b.st[s];
-  if (!st.active || !st.nl_invalid) return;
-  st.nl_invalid = 0;
-  st.rebuilds += 1;
+  const bool inv = st.active && st.nl_invalid;
+  __syncthreads();
+  if (!inv) return;
+  clear_cells(b, b.sys[s], threadIdx.x, blockDim.x);
+  if (threadIdx.x == 0) {
+    st.nl_invalid = 0;
+    st.rebuilds += 1;
+  }
 }
 
 // ------------------------------------------------------------------ terms ----
-// Every enabled term in one launch: blockIdx.z is the term, blockIdx.y the
+// Forces accumulate in FP64 in every precision: FP64 atomics cost the L2 what
+// FP32 ones do.
+
+// A single term, as the host's per-term calls ask for it: blockIdx.y is the
 // system, blockIdx.x strides over the term's list.
-template <typename R, typename RF> __global__ void k_terms(DevBatch b, int only_term, int from, int to) {
-  int term = only_term >= 0 ? only_term : (int)blockIdx.z;
+template <typename R> __global__ void k_terms(DevBatch b, int term, int from, int to) {
   int s = blockIdx.y;
   SysState &st = b.st[s];
   if (!st.active || !term_on(*b.P, term)) return;
@@ -614,12 +606,180 @@ template <typename R, typename RF> __global__ void k_terms(DevBatch b, int only_
   int n = term_size(sd, st, term);
   int lo = from > 0 ? from : 0, hi = (to >= 0 && to < n) ? to : n;
   GeoG g{b.y[0][0], b.y[0][1], b.y[0][2]};
-  AccG<RF> acc{(RF *)b.F[0], (RF *)b.F[1], (RF *)b.F[2]};
+  AccG acc{b.acc[0], b.acc[1], b.acc[2]};
   double v = 0.0;
   for (int k = lo + blockIdx.x * blockDim.x + threadIdx.x; k < hi; k += gridDim.x * blockDim.x)
     v += eval_item<R>(b, sd, st, g, acc, term, k, st.t);
   v = block_sum(v);
   if (threadIdx.x == 0 && v != 0.0) atomicAdd(&st.V[term], v);
+}
+
+// The sum of v over the wave in lane 63: row shifts within 16 lanes, then the
+// rows' totals broadcast along (a DPP move is one vector instruction; a
+// cross-lane shuffle an LDS round trip).
+template <int CTRL, int ROWS> __device__ __forceinline__ double dpp_add(double v) {
+  const long long x = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, ROWS, 0xf, true);
+  return v + __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+__device__ __forceinline__ double wave_total(double v) {
+  v = dpp_add<0x111, 0xf>(v);
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+__device__ __forceinline__ void add_energy(SysState &st, int term, double v) {
+  v = wave_total(v);
+  if ((threadIdx.x & 63) == 63 && v != 0.0) atomicAdd(&st.V[term], v);
+}
+
+// 64 base residues' chain-local bonded items (bond_regular): every lane
+// evaluates the items that start at its residue, in FP64 as eval_item does,
+// from one read of its four residues; a residue's force is its own share plus
+// those lanes 1..3 below computed for it, so a residue takes 3 atomics a group
+// where its items would take 9 or 12 each. Shares past the wave's last lane go
+// out directly. The items fall into three groups for different waves, as one
+// wave's chain of all seven would be the step's longest.
+enum { BG_DIH, BG_CHIR, BG_SHORT, BG_N };
+template <int GROUP>
+__device__ __forceinline__ void bonded_chunk(const DevBatch &b, SysDescC &sd, SysState &st,
+                                             const GeoG &g, AccG &acc, int chunk) {
+  ParamsC &p = b.P->p;
+  const int lane = threadIdx.x & 63, k = chunk * 64 + lane, last = sd.res0 + sd.n - 1;
+  const bool mine = k < sd.n;
+  const int r = min(sd.res0 + k, last);
+  GeoR q;
+  q.base = r;
+  for (int j = 0; j < 4; ++j) q.p[j] = g.r(min(r + j, last));
+  AccSlots<double> a;
+  a.base = r;
+  for (int s = 0; s < 4; ++s) a.c[s][0] = a.c[s][1] = a.c[s][2] = 0.0;
+  const int variant = p.nat_dih_variant;
+  auto part = [&](int term, int L, auto item) {
+    const int t = mine ? b.bond_item[L][r] : -1;
+    if (!__any(t >= 0)) return;
+    double v = 0.0;
+    if (t >= 0) v = item(t);
+    add_energy(st, term, v);
+  };
+  if (GROUP == BG_SHORT) {
+    part(PCG_TETHER, BOND_TETHER,
+         [&](int t) { return tether_core<double>(p, q, a, r, r + 1, b.teth_nat[t]); });
+    part(PCG_LREP, BOND_LREP, [&](int) { return lrep_core<double>(p, q, a, r, r + 2); });
+    part(PCG_NAT_ANG, BOND_NAT_ANG,
+         [&](int t) { return nat_ang_core<double>(p, q, a, r, r + 1, r + 2, b.nang_th[t]); });
+    part(PCG_HEUR_ANG, BOND_HEUR_ANG,
+         [&](int t) { return heur_ang_core<double>(p, q, a, r, r + 1, r + 2, b.hang_t[t]); });
+  } else if (GROUP == BG_DIH) {
+    part(variant ? PCG_SND : PCG_CND, BOND_NAT_DIH, [&](int t) {
+      const double phi0 = b.ndih_ph[t];
+      double s0 = 0.0, c0 = 1.0;
+      if (variant == 0) sincos(phi0, &s0, &c0);
+      return nat_dih_core<double>(p, q, a, r, r + 1, r + 2, r + 3, phi0, c0, s0, variant);
+    });
+    part(PCG_HEUR_DIH, BOND_HEUR_DIH, [&](int t) {
+      return heur_dih_core<double>(p, q, a, r, r + 1, r + 2, r + 3, b.hdih_t[t]);
+    });
+  } else {
+    part(PCG_CHIR, BOND_CHIR, [&](int t) {
+      return chir_core<double>(p, q, a, r, r + 1, r + 2, r + 3, b.chir_f0[t], b.chir_f1[t]);
+    });
+  }
+  double f[3];
+  for (int c = 0; c < 3; ++c) {
+    const double s1 = __shfl_up(a.c[1][c], 1, 64), s2 = __shfl_up(a.c[2][c], 2, 64),
+                 s3 = __shfl_up(a.c[3][c], 3, 64);
+    f[c] = a.c[0][c];
+    if (lane >= 1) f[c] += s1;
+    if (lane >= 2) f[c] += s2;
+    if (lane >= 3) f[c] += s3;
+  }
+  if (!mine) return;
+  acc.add(r, v3<double>{f[0], f[1], f[2]});
+  for (int s = 1; s < 4; ++s)
+    if (lane + s >= 64 && (a.c[s][0] != 0.0 || a.c[s][1] != 0.0 || a.c[s][2] != 0.0))
+      acc.add(r + s, v3<double>{a.c[s][0], a.c[s][1], a.c[s][2]});
+}
+
+template <int T> struct Term {
+  static constexpr int value = T;
+};
+// Every enabled term of a step in one launch: blockIdx.y is the system, whose
+// waves stride over the 64-item chunks of all its terms, the long chains of
+// bonded items first. Each wave finds its chunk from the list sizes on the
+// device, so the grid follows the work. A wave's chunk is a serial chain of
+// some thousand instructions on almost empty SIMDs, which bounds the kernel: a
+// grid of blocks for every term at its largest size was 11 000 blocks, nearly
+// all empty, and took 17.4 us for a box of 6400 residues, 18 for 2000 in one
+// chain and 13.1 for 480 between walls; this one takes 13.2, 15.7 and 11.1
+// (29 and more with one chunk of all the bonded items). Also resets what the
+// step's verify read.
+template <typename R> __global__ __launch_bounds__(BLK) void k_step_terms(DevBatch b, int step) {
+  const int s = blockIdx.y;
+  SysState &st = b.st[s];
+  if (!st.active) return;
+  SysDescC &sd = b.sys[s];
+  const int nwaves = gridDim.x * (BLK / 64);
+  const int w0 = __builtin_amdgcn_readfirstlane(blockIdx.x * (BLK / 64) + (threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  if (step && st.nl_invalid) clear_cells(b, sd, w0 * 64 + lane, nwaves * 64);
+  if (step && blockIdx.x == 0 && threadIdx.x == 0) {
+    st.max_disp_bits = 0ull;
+    if (b.P->nl_required) st.verify_first = 0;
+  }
+  GeoG g{b.y[0][0], b.y[0][1], b.y[0][2]};
+  AccG acc{b.acc[0], b.acc[1], b.acc[2]};
+  const double t = st.t;
+  for (int w = w0;; w += nwaves) {
+    int c = w;  // the wave's chunk, counted down through the terms
+    // (uniform) chunk c of term T, or past its end
+    auto term = [&](auto tag) -> bool {
+      constexpr int T = decltype(tag)::value;
+      if (!term_on(*b.P, T)) return false;
+      const int n = __builtin_amdgcn_readfirstlane(term_size(sd, st, T)), chunks = (n + 63) >> 6;
+      if (c >= chunks) {
+        c -= chunks;
+        return false;
+      }
+      const int k = c * 64 + lane;
+      double v = 0.0;
+      if (k < n) v = eval_item<R>(b, sd, st, g, acc, T, k, t);
+      add_energy(st, T, v);
+      return true;
+    };
+    if (sd.bond_regular) {
+      const int chunks = (sd.n + 63) >> 6;
+      // chunk c of a group with items
+      auto group = [&](auto tag, bool any) -> bool {
+        if (!any) return false;
+        if (c >= chunks) {
+          c -= chunks;
+          return false;
+        }
+        bonded_chunk<decltype(tag)::value>(b, sd, st, g, acc, c);
+        return true;
+      };
+      if (group(Term<BG_DIH>(), sd.nndih > 0 || sd.nhdih > 0) ||
+          group(Term<BG_CHIR>(), sd.nchir > 0) ||
+          group(Term<BG_SHORT>(), sd.nteth > 0 || sd.nlrep > 0 || sd.nnang > 0 || sd.nhang > 0))
+        continue;
+    } else if (term(Term<PCG_CHIR>()) || term(Term<PCG_TETHER>()) || term(Term<PCG_LREP>()) ||
+               term(Term<PCG_NAT_ANG>()) || term(Term<PCG_HEUR_ANG>()) ||
+               term(Term<PCG_HEUR_DIH>()) || term(Term<PCG_CND>()) || term(Term<PCG_SND>())) {
+      continue;
+    }
+    if (term(Term<PCG_QA_CONT>()) || term(Term<PCG_NAT_CONT>()) || term(Term<PCG_PID>()) ||
+        term(Term<PCG_QA_CAND>()) || term(Term<PCG_PAULI>()) || term(Term<PCG_CONST_DH>()) ||
+        term(Term<PCG_REL_DH>()) || term(Term<PCG_VEL_AFM>()) || term(Term<PCG_FORCE_AFM>()) ||
+        term(Term<PCG_SOLID_WALL>()) || term(Term<PCG_HW_FREE>()) || term(Term<PCG_HW_CONN>()) ||
+        term(Term<PCG_LJW_FREE>()) || term(Term<PCG_LJW_CONN>()))
+      continue;
+    break;
+  }
 }
 
 // ------------------------------------------------------------------- QA ----
@@ -629,26 +789,6 @@ __global__ void k_prepare_nh(DevBatch b) {
   if (!b.st[b.sysid[i]].active) return;
   GeoG g{b.y[0][0], b.y[0][1], b.y[0][2]};
   prepare_nh_item(b, g, i);
-}
-
-// The first kernel of a full step, over residues: each system's first
-// residue runs the system's begin (energies and the walls' reaction forces
-// cleared, nl::verify), every residue clears its force and, with QA on,
-// computes its n and h (k_begin, the force clearing and k_prepare_nh in one
-// launch; none reads what another writes)
-template <typename RF> __global__ void k_step_begin(DevBatch b, int qa_on) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= b.ntot) return;
-  const int s = b.sysid[i];
-  if (b.local[i] == 0) begin_system(b, s);
-  if (!b.st[s].active) return;
-  ((RF *)b.F[0])[i] = 0;
-  ((RF *)b.F[1])[i] = 0;
-  ((RF *)b.F[2])[i] = 0;
-  if (qa_on) {
-    GeoG g{b.y[0][0], b.y[0][1], b.y[0][2]};
-    prepare_nh_item(b, g, i);
-  }
 }
 
 // The serial part of the finish (removals, then acceptance in order) reads
@@ -686,38 +826,91 @@ __global__ void k_qa_finish(DevBatch b, int sync_lds) {
   for (int k = threadIdx.x; k < n; k += blockDim.x) *(uint32_t *)(b.sync + 4 * (r0 + k)) = syl[k];
 }
 
-// time and energy bookkeeping at the end of a step (step.cpp:157-162)
-__device__ __forceinline__ void tick_system(const DevBatch &b, int s, int advance, int nl_done) {
-  SysState &st = b.st[s];
-  // a full step's rebuild, if it made one, is complete (k_nl_done)
-  if (nl_done && st.nl_invalid) {
-    st.nl_invalid = 0;
-    st.rebuilds += 1;
+// wall::log_forces (cg/src/cg/wall/log_forces.cpp:4-17) after the forces of
+// a step: every plane on a box side, then once more the -axis plane of each
+// LJ axis (the reference's wall list holds it twice, state.cpp:680-681);
+// work += F . shift; the z force averaged. One thread a side, as the planes
+// keep apart, and one for the z force (threads 0..6; by one thread in turn the
+// log took 5.6 us of the 44 a 480-residue box step ran).
+__device__ __forceinline__ void box_log(const DevBatch &b) {
+#pragma clang fp contract(off)
+  WallDev &W = *b.wall;
+  const SysState &st = b.st[0];
+  if (!st.active || !W.log_on) return;
+  ParamsC &p = b.P->p;
+  const double t = st.t;
+  auto one = [&](int w) {
+    mavg_add(W.avg_F[w], t, W.wall_F[w], 3);
+    W.work[w] += W.wall_F[w][0] * W.shift[w][0] + W.wall_F[w][1] * W.shift[w][1] +
+                 W.wall_F[w][2] * W.shift[w][2];
+  };
+  const int side = threadIdx.x;
+  if (side < 6) {
+    const int w = W.side_wall[side];
+    if (w >= 0) one(w);
+    if (w >= 0 && (side & 1) == 0 && p.wall_kind[w] == 2) one(w);
   }
+  if (side != 6) return;
+  const int wn = W.side_wall[4], wp = W.side_wall[5];
+  const double zf = (W.wall_F[wn][0] * p.wall_normal[wn][0] + W.wall_F[wn][1] * p.wall_normal[wn][1] +
+                     W.wall_F[wn][2] * p.wall_normal[wn][2]) +
+                    (W.wall_F[wp][0] * p.wall_normal[wp][0] + W.wall_F[wp][1] * p.wall_normal[wp][1] +
+                     W.wall_F[wp][2] * p.wall_normal[wp][2]);
+  mavg_add(W.avg_z, t, &zf, 1);
+}
+
+// time and energy bookkeeping at the end of a step (step.cpp:157-162)
+// v: the sum of its energies
+__device__ __forceinline__ void tick_system(const DevBatch &b, int s, int advance, int nl_done,
+                                            double v) {
+  SysState &st = b.st[s];
+  // (all reads first: one wait instead of one for each)
+  const int invalid = st.nl_invalid, rebuilds = st.rebuilds, overflow = st.overflow;
+  const double t = st.true_t + b.P->dt;
+  const auto step = st.step;
+  const int lang = b.P->p.lang_on;
+  // a full step's rebuild, if it made one, is complete (k_nl_done)
+  if (nl_done && invalid) {
+    st.nl_invalid = 0;
+    st.rebuilds = rebuilds + 1;
+  }
+  st.Vtot = v;
+  if (b.ovf && overflow) *b.ovf = 1;
+  if (advance && lang) {
+    st.true_t = t;
+    st.t = t;
+    st.step = step + 1;
+  }
+}
+__device__ __forceinline__ double sum_energies(const SysState &st) {
   double v = 0.0;
   for (int k = 0; k < NT; ++k) v += st.V[k];
-  st.Vtot = v;
-  if (b.ovf && st.overflow) *b.ovf = 1;
-  if (advance && b.P->p.lang_on) {
-    st.true_t += b.P->dt;
-    st.t = st.true_t;
-    st.step += 1;
-  }
+  return v;
 }
 
 __global__ void k_tick(DevBatch b, int advance, int nl_done) {
   int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= b.nsys) return;
   if (!b.st[s].active) return;
-  tick_system(b, s, advance, nl_done);
+  tick_system(b, s, advance, nl_done, sum_energies(b.st[s]));
 }
 
 
 // The displacement maximum goes to the system's state with one atomic per
 // wave when the wave's residues belong to one system (a system of the plain
 // context has thousands of residues: one atomic per residue on one address
-// serialised the whole kernel), else one per residue.
-template <typename RF> __global__ void k_lang(DevBatch b, int noise_mode, int tick) {
+// serialised the whole kernel), else one per residue. The forces come from the
+// FP64 accumulators and go to the force arrays in their precision.
+//
+// The step's tick is run by the wave that completes its system. It waits for
+// no other wave's results, only for every wave to have read the time and step
+// it advances, which a wave has when it counts itself: so the count needs no
+// fence (an agent-scope one writes back the L2; 8.8 us with it, 7.9 without,
+// for 6400 residues). What the tick adds up is
+// read before the count, as it is final by then. log (one system): one more
+// block than the residues need keeps the wall forces' log, which reads the
+// time too, and counts itself as one more item.
+template <typename RF> __global__ void k_lang(DevBatch b, int noise_mode, int tick, int log) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   int s = -1, sys = -1;
   bool mine = false;   // a residue of an active system
@@ -736,14 +929,23 @@ template <typename RF> __global__ void k_lang(DevBatch b, int noise_mode, int ti
       } else {
         philox_normals(sd.philox_key, st.step, b.local[i], nz);
       }
+      const double F[3] = {b.acc[0][i], b.acc[1][i], b.acc[2][i]};
       double r[3];
-      gear_update(b, sd, st, i, (double)((RF *)b.F[0])[i], (double)((RF *)b.F[1])[i],
-                  (double)((RF *)b.F[2])[i], nz, r);
+      gear_update(b, sd, st, i, F[0], F[1], F[2], nz, r);
+      if (sizeof(RF) == 4)
+        for (int c = 0; c < 3; ++c) ((RF *)b.F[c])[i] = (RF)F[c];
       disp = disp_from_orig(b, sd, i, r);
     } else {
       s = -1;
     }
+  } else if (log && blockIdx.x == gridDim.x - 1 && threadIdx.x < 7) {
+    mine = threadIdx.x == 0 && b.st[0].active != 0;
+    sys = 0;
+    box_log(b);
   }
+  // the energies of the wave's first system, one a lane, for the tick
+  const int sys0 = __shfl(sys, 0, 64), lane = threadIdx.x & 63;
+  const double vk = tick && sys0 >= 0 && lane < NT ? b.st[sys0].V[lane] : 0.0;
   const int s0 = __shfl(s, 0, 64);
   if (__all(s == s0)) {
     double m = disp;
@@ -753,13 +955,13 @@ template <typename RF> __global__ void k_lang(DevBatch b, int noise_mode, int ti
   } else if (s >= 0) {
     atomicMax(&b.st[s].max_disp_bits, (unsigned long long)__double_as_longlong(disp));
   }
-  // the step's tick (k_tick) by the residue that completes its system, once
-  // every residue's Langevin work, and with it every read of the system's
-  // time, is done
   if (tick) {
-    const int done = count_done(b, &SysState::done_lang, mine, sys);
+    const int done = count_done(b, &SysState::done_lang, mine, sys, false, log);
+    double v = 0.0;
+    if (__any(done >= 0))
+      for (int k = 0; k < NT; ++k) v += __shfl(vk, k, 64);
     if (done >= 0) {
-      tick_system(b, done, 1, 1);
+      tick_system(b, done, 1, 1, done == sys0 ? v : sum_energies(b.st[done]));
       b.st[done].done_lang = 0;
     }
   }
@@ -1078,48 +1280,20 @@ __global__ void k_box_phase(DevBatch b, DevParams *P, SysDesc *sd) {
   }
 }
 
-// wall::log_forces (cg/src/cg/wall/log_forces.cpp:4-17) after the forces of
-// a step: every plane on a box side, then once more the -axis plane of each
-// LJ axis (the reference's wall list holds it twice, state.cpp:680-681);
-// work += F . shift; the z force averaged
-__global__ void k_box_log(DevBatch b) {
-#pragma clang fp contract(off)
-  if (threadIdx.x != 0) return;
-  WallDev &W = *b.wall;
-  const SysState &st = b.st[0];
-  if (!st.active || !W.log_on) return;
-  ParamsC &p = b.P->p;
-  const double t = st.t;
-  auto one = [&](int w) {
-    mavg_add(W.avg_F[w], t, W.wall_F[w], 3);
-    W.work[w] += W.wall_F[w][0] * W.shift[w][0] + W.wall_F[w][1] * W.shift[w][1] +
-                 W.wall_F[w][2] * W.shift[w][2];
-  };
-  for (int side = 0; side < 6; ++side)
-    if (W.side_wall[side] >= 0) one(W.side_wall[side]);
-  for (int side = 0; side < 6; side += 2) {
-    const int w = W.side_wall[side];
-    if (w >= 0 && p.wall_kind[w] == 2) one(w);
-  }
-  const int wn = W.side_wall[4], wp = W.side_wall[5];
-  const double zf = (W.wall_F[wn][0] * p.wall_normal[wn][0] + W.wall_F[wn][1] * p.wall_normal[wn][1] +
-                     W.wall_F[wn][2] * p.wall_normal[wn][2]) +
-                    (W.wall_F[wp][0] * p.wall_normal[wp][0] + W.wall_F[wp][1] * p.wall_normal[wp][1] +
-                     W.wall_F[wp][2] * p.wall_normal[wp][2]);
-  mavg_add(W.avg_z, t, &zf, 1);
-}
-
 // ------------------------------------------------------------- launchers ----
 static inline dim3 grid1(int n, int blk = BLK) { return dim3((unsigned)((n + blk - 1) / blk)); }
 
 void launch_begin(const DevBatch &b, hipStream_t s) {
   hipLaunchKernelGGL(k_begin, grid1(b.nsys, 64), dim3(64), 0, s, b);
 }
-void launch_eval_begin(const DevBatch &b, int prec, hipStream_t s) {
-  if (prec == PCG_FP64)
-    hipLaunchKernelGGL(k_eval_begin<double>, grid1(b.ntot), dim3(BLK), 0, s, b);
-  else
-    hipLaunchKernelGGL(k_eval_begin<float>, grid1(b.ntot), dim3(BLK), 0, s, b);
+void launch_eval_begin(const DevBatch &b, hipStream_t s) {
+  hipLaunchKernelGGL(k_eval_begin, grid1(b.ntot), dim3(BLK), 0, s, b);
+}
+void launch_store_forces(const DevBatch &b, hipStream_t s) {
+  hipLaunchKernelGGL(k_move_forces<true>, grid1(b.ntot), dim3(BLK), 0, s, b);
+}
+void launch_load_forces(const DevBatch &b, hipStream_t s) {
+  hipLaunchKernelGGL(k_move_forces<false>, grid1(b.ntot), dim3(BLK), 0, s, b);
 }
 void launch_mark_invalid(const DevBatch &b, hipStream_t s) {
   hipLaunchKernelGGL(k_mark_invalid, grid1(b.nsys, 64), dim3(64), 0, s, b);
@@ -1130,12 +1304,13 @@ void launch_fetch(const Fetch &f, hipStream_t s) {
   if (f.f32)
     hipLaunchKernelGGL(k_fetch<float>, dim3(1), block, 0, s, (const uint32_t *)f.src,
                        (uint32_t *)f.dst, (int)(f.bytes / 4), (const float *)f.cols[0],
-                       (const float *)f.cols[1], (const float *)f.cols[2], f.out, f.n, f.flag, f.seq);
+                       (const float *)f.cols[1], (const float *)f.cols[2], f.acc, f.out, f.n, f.flag,
+                       f.seq);
   else
     hipLaunchKernelGGL(k_fetch<double>, dim3(1), block, 0, s, (const uint32_t *)f.src,
                        (uint32_t *)f.dst, (int)(f.bytes / 4), (const double *)f.cols[0],
-                       (const double *)f.cols[1], (const double *)f.cols[2], f.out, f.n, f.flag,
-                       f.seq);
+                       (const double *)f.cols[1], (const double *)f.cols[2], (const double *)nullptr, f.out, f.n,
+                       f.flag, f.seq);
 }
 void launch_noise_in(const DevBatch &b, const double *src, hipStream_t s) {
   hipLaunchKernelGGL(k_noise_in, grid1(b.ntot), dim3(BLK), 0, s, b, src);
@@ -1143,45 +1318,46 @@ void launch_noise_in(const DevBatch &b, const double *src, hipStream_t s) {
 void launch_prepare_nh(const DevBatch &b, hipStream_t s) {
   hipLaunchKernelGGL(k_prepare_nh, grid1(b.ntot), dim3(BLK), 0, s, b);
 }
-void launch_step_begin(const DevBatch &b, int prec, int qa_on, hipStream_t s) {
-  if (prec == PCG_FP64)
-    hipLaunchKernelGGL(k_step_begin<double>, grid1(b.ntot), dim3(BLK), 0, s, b, qa_on);
-  else
-    hipLaunchKernelGGL(k_step_begin<float>, grid1(b.ntot), dim3(BLK), 0, s, b, qa_on);
-}
-void launch_fix_nl(const DevBatch &b, int max_n, int max_nlcap, int cell_words, hipStream_t s,
-                   bool done) {
+void launch_fix_nl(const DevBatch &b, int max_n, int cell_words, hipStream_t s, bool step,
+                   int qa_on) {
   int rows_per_block = BLK / 64;
   dim3 rg((unsigned)((b.ntot + rows_per_block - 1) / rows_per_block));
   const size_t mask_lds = (size_t)rows_per_block * cell_words * sizeof(unsigned long long);
-  // each count kernel ends with the scan of its counts, by the wave or
-  // block that completes a system
-  if (cell_words > 0) {
-    hipLaunchKernelGGL(k_cell_count, grid1(b.ntot), dim3(BLK), 0, s, b);
+  const int begin = step ? 1 : 0, cells = cell_words > 0;
+  // the cell counts and, for smaller systems, the row counts are scanned by
+  // the wave that completes them
+  if (cells) {
+    hipLaunchKernelGGL(k_cell_count, grid1(b.ntot), dim3(BLK), 0, s, b, begin, qa_on);
     hipLaunchKernelGGL(k_cell_fill, grid1(b.ntot), dim3(BLK), 0, s, b);
   }
   const int fuse = max_n < ROWS_FUSE_MAX;
-  hipLaunchKernelGGL(k_nl_rows<false>, rg, dim3(BLK), mask_lds, s, b, cell_words, fuse);
-  if (!fuse) hipLaunchKernelGGL(k_nl_scan, dim3((unsigned)b.nsys), dim3(64), 0, s, b);
-  hipLaunchKernelGGL(k_nl_rows<true>, rg, dim3(BLK), mask_lds, s, b, cell_words, fuse);
-  // the partition strides over the filled chunks: at most PART_GRID blocks
-  // a system (one per CU of a 256-CU device for one system)
-  const int part_grid = std::max(1, std::min((max_nlcap + BLK - 1) / BLK, PART_GRID));
-  dim3 pg((unsigned)part_grid, (unsigned)b.nsys);
-  hipLaunchKernelGGL(k_part_count, pg, dim3(BLK), 0, s, b);
-  hipLaunchKernelGGL(k_part_write, pg, dim3(BLK), 0, s, b);
-  if (done) hipLaunchKernelGGL(k_nl_done, grid1(b.nsys, 64), dim3(64), 0, s, b);
+  hipLaunchKernelGGL(k_nl_rows<false>, rg, dim3(BLK), mask_lds, s, b, cell_words, fuse,
+                     cells ? 0 : begin, qa_on);
+  if (!fuse) hipLaunchKernelGGL(k_nl_scan, dim3((unsigned)b.nsys), dim3(64 * (RC_N + 1)), 0, s, b);
+  hipLaunchKernelGGL(k_nl_rows<true>, rg, dim3(BLK), mask_lds, s, b, cell_words, fuse, 0, 0);
+  if (!step) hipLaunchKernelGGL(k_nl_done, dim3((unsigned)b.nsys), dim3(BLK), 0, s, b);
 }
-void launch_terms(const DevBatch &b, int prec, int max_items, int only_term, int from, int to,
+void launch_terms(const DevBatch &b, int prec, int max_items, int term, int from, int to,
                   hipStream_t s) {
   int gx = (max_items + BLK - 1) / BLK;
   if (gx < 1) gx = 1;
   if (gx > 512) gx = 512;
-  dim3 g((unsigned)gx, (unsigned)b.nsys, only_term >= 0 ? 1u : (unsigned)NT);
+  dim3 g((unsigned)gx, (unsigned)b.nsys);
   if (prec == PCG_FP64)
-    hipLaunchKernelGGL((k_terms<double, double>), g, dim3(BLK), 0, s, b, only_term, from, to);
+    hipLaunchKernelGGL(k_terms<double>, g, dim3(BLK), 0, s, b, term, from, to);
   else
-    hipLaunchKernelGGL((k_terms<float, float>), g, dim3(BLK), 0, s, b, only_term, from, to);
+    hipLaunchKernelGGL(k_terms<float>, g, dim3(BLK), 0, s, b, term, from, to);
+}
+void launch_step_terms(const DevBatch &b, int prec, int max_n, bool step, hipStream_t s) {
+  // a wave for some four residues: the chunks of the usual force field (bonded
+  // n / 64, native contacts and QA near pairs n / 4 and more); longer lists
+  // stride. At most eight waves a SIMD of the chip.
+  const int gx = std::max(16, std::min((max_n / 4 + 3) / 4, 2048));
+  dim3 g((unsigned)gx, (unsigned)b.nsys);
+  if (prec == PCG_FP64)
+    hipLaunchKernelGGL(k_step_terms<double>, g, dim3(BLK), 0, s, b, step ? 1 : 0);
+  else
+    hipLaunchKernelGGL(k_step_terms<float>, g, dim3(BLK), 0, s, b, step ? 1 : 0);
 }
 size_t qa_finish_lds(int max_n) {
   return 4 * (((size_t)max_n + 1) & ~(size_t)1) + (size_t)QF_CAND_LDS * (8 + 8 + 4 * 4);
@@ -1192,12 +1368,14 @@ void launch_qa_finish(const DevBatch &b, int max_n, hipStream_t s) {
   const int sync_lds = lds <= QF_LDS_MAX ? max_n : 0;
   hipLaunchKernelGGL(k_qa_finish, dim3(b.nsys), dim3(1024), sync_lds ? lds : 0, s, b, sync_lds);
 }
-void launch_lang(const DevBatch &b, int prec, int noise_mode, hipStream_t s, bool tick) {
-  const int t = tick ? 1 : 0;
+void launch_lang(const DevBatch &b, int prec, int noise_mode, hipStream_t s, bool tick, bool log) {
+  const int t = tick ? 1 : 0, l = log ? 1 : 0;
+  dim3 g = grid1(b.ntot);
+  g.x += l;
   if (prec == PCG_FP64)
-    hipLaunchKernelGGL(k_lang<double>, grid1(b.ntot), dim3(BLK), 0, s, b, noise_mode, t);
+    hipLaunchKernelGGL(k_lang<double>, g, dim3(BLK), 0, s, b, noise_mode, t, l);
   else
-    hipLaunchKernelGGL(k_lang<float>, grid1(b.ntot), dim3(BLK), 0, s, b, noise_mode, t);
+    hipLaunchKernelGGL(k_lang<float>, g, dim3(BLK), 0, s, b, noise_mode, t, l);
 }
 void launch_tick(const DevBatch &b, int advance, hipStream_t s, bool nl_done) {
   hipLaunchKernelGGL(k_tick, grid1(b.nsys, 64), dim3(64), 0, s, b, advance, nl_done ? 1 : 0);
@@ -1211,8 +1389,4 @@ void launch_box_setup(const DevBatch &b, DevParams *P, SysDesc *sd, hipStream_t 
 void launch_box_phase(const DevBatch &b, DevParams *P, SysDesc *sd, hipStream_t s) {
   hipLaunchKernelGGL(k_box_phase, dim3(1), dim3(64), 0, s, b, P, sd);
 }
-void launch_box_log(const DevBatch &b, hipStream_t s) {
-  hipLaunchKernelGGL(k_box_log, dim3(1), dim3(64), 0, s, b);
-}
-
 } // namespace pcg

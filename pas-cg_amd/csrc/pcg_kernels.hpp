@@ -8,8 +8,6 @@
 namespace pcg {
 
 constexpr int BLK = 256;
-// most blocks a system's partition kernels take (they stride over the chunks)
-constexpr int PART_GRID = 256;
 // systems of this many residues or more take the NL row scan as a launch of
 // its own (k_nl_scan) instead of in the count pass's last row
 constexpr int ROWS_FUSE_MAX = 2048;
@@ -36,12 +34,12 @@ struct GeoG {
   }
 };
 
-template <typename RF> struct AccG {
-  RF *fx, *fy, *fz;
+struct AccG {
+  double *fx, *fy, *fz;
   template <typename T> __device__ __forceinline__ void add(int i, v3<T> f) {
-    atomicAdd(fx + i, (RF)f.x);
-    atomicAdd(fy + i, (RF)f.y);
-    atomicAdd(fz + i, (RF)f.z);
+    atomicAdd(fx + i, (double)f.x);
+    atomicAdd(fy + i, (double)f.y);
+    atomicAdd(fz + i, (double)f.z);
   }
 };
 

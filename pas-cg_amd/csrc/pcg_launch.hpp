@@ -6,16 +6,23 @@
 namespace pcg {
 void launch_begin(const DevBatch &b, hipStream_t s);
 // forces, energies and wall reactions to zero before an evaluation outside a step
-void launch_eval_begin(const DevBatch &b, int prec, hipStream_t s);
+void launch_eval_begin(const DevBatch &b, hipStream_t s);
+// the FP64 force accumulators into FP32 force arrays
+void launch_store_forces(const DevBatch &b, hipStream_t s);
+// and back
+void launch_load_forces(const DevBatch &b, hipStream_t s);
 void launch_mark_invalid(const DevBatch &b, hipStream_t s);
 // device data into mapped pinned host memory: bytes of src as words, and three
-// columns of n values (FP32 or FP64) as FP64 triples; then seq into flag
+// columns of n values (FP32 or FP64) as FP64 triples; then seq into flag. acc
+// (with f32): the columns are forces still in these accumulators, n of each
+// component, and are stored on the way.
 struct Fetch {
   const void *src = nullptr;
   void *dst = nullptr;
   size_t bytes = 0;
   const void *cols[3] = {nullptr, nullptr, nullptr};
   bool f32 = false;
+  const double *acc = nullptr;
   int n = 0;
   double *out = nullptr;
   int *flag = nullptr;  // null: no flag
@@ -25,25 +32,29 @@ void launch_fetch(const Fetch &f, hipStream_t s);
 // the host's noise of one step into the device's
 void launch_noise_in(const DevBatch &b, const double *src, hipStream_t s);
 void launch_prepare_nh(const DevBatch &b, hipStream_t s);
-// begin, force clearing and (qa_on) prepare_nh of a full step in one launch
-void launch_step_begin(const DevBatch &b, int prec, int qa_on, hipStream_t s);
-// done: close the rebuild here (else the step's k_tick does, nl_done)
-void launch_fix_nl(const DevBatch &b, int max_n, int max_nlcap, int cell_words, hipStream_t s,
-                   bool done = true);
-void launch_terms(const DevBatch &b, int prec, int max_items, int only_term, int from, int to,
+// The list rebuild of every system that needs one. step: the first kernels of
+// a full step, which also take the verify decision, clear the forces and
+// energies and (qa_on) compute n and h; else the systems marked invalid, and
+// the rebuild is closed here.
+void launch_fix_nl(const DevBatch &b, int max_n, int cell_words, hipStream_t s, bool step,
+                   int qa_on);
+// every term, of a step or (step false) of an evaluation outside one
+void launch_step_terms(const DevBatch &b, int prec, int max_n, bool step, hipStream_t s);
+// a single term outside a step
+void launch_terms(const DevBatch &b, int prec, int max_items, int term, int from, int to,
                   hipStream_t s);
 void launch_qa_finish(const DevBatch &b, int max_n, hipStream_t s);
-// tick: the step's k_tick (advance, close a rebuild) by the residue that
-// completes each system
-void launch_lang(const DevBatch &b, int prec, int noise_mode, hipStream_t s, bool tick = false);
+// tick: the step's k_tick (advance, close a rebuild) by the wave that
+// completes each system, log: after the wall forces' log of the box protocol
+void launch_lang(const DevBatch &b, int prec, int noise_mode, hipStream_t s, bool tick = false,
+                 bool log = false);
 void launch_tick(const DevBatch &b, int advance, hipStream_t s, bool nl_done = false);
 // walls and the box protocol of a plain context (b.wall set): LJ candidate
-// processing; box set-up, the phase logic before a step, the force log after
-// it. P and sd are the writable device parameters and system descriptor.
+// processing; box set-up, and the phase logic before a step. P and sd are the
+// writable device parameters and system descriptor.
 void launch_ljw_process(const DevBatch &b, hipStream_t s);
 void launch_box_setup(const DevBatch &b, DevParams *P, SysDesc *sd, hipStream_t s);
 void launch_box_phase(const DevBatch &b, DevParams *P, SysDesc *sd, hipStream_t s);
-void launch_box_log(const DevBatch &b, hipStream_t s);
 // persistent form: every system of the batch advances nsteps in one launch;
 // lean: the lean kernels (pcg_batch_lean.hip), for batches lean_batch allows
 void launch_persistent(const DevBatch &b, bool lean, int prec, int block, int nsteps,

@@ -675,22 +675,6 @@ __device__ __forceinline__ void wg_fix_nl(DevBatchC *bp, int s, SysState &st, co
   __syncthreads();
 }
 
-// Shares of one chain-local item: slot s receives the force on residue
-// base + s (s = 0..3), in registers.
-template <typename RF> struct AccSlots {
-  int base;
-  RF c[4][3];
-  template <typename T> __device__ __forceinline__ void add(int i, v3<T> f) {
-    int s = i - base;
-    // explicit selects keep c in registers
-    RF fx = (RF)f.x, fy = (RF)f.y, fz = (RF)f.z;
-    if (s == 0) { c[0][0] += fx; c[0][1] += fy; c[0][2] += fz; }
-    else if (s == 1) { c[1][0] += fx; c[1][1] += fy; c[1][2] += fz; }
-    else if (s == 2) { c[2][0] += fx; c[2][1] += fy; c[2][2] += fz; }
-    else { c[3][0] += fx; c[3][1] += fy; c[3][2] += fz; }
-  }
-};
-
 // Per-residue bonded parameters of a chain-local system in LDS: the item
 // starting at residue k of each list exists if its flag bit is set.
 enum { BF_TETHER = 1, BF_LREP = 2, BF_NAT_ANG = 4, BF_HEUR_ANG = 8, BF_NAT_DIH = 16,
@@ -747,14 +731,6 @@ __device__ __forceinline__ void stage_bonded(const DevBatch &b, SysDescC &sd, co
 template <typename RF> __device__ __forceinline__ RF shfl_up_rf(RF v, int d) {
   return __shfl_up(v, (unsigned)d, 64);
 }
-
-// The four residues of a base residue's items, read from LDS once for all of
-// them (past the chain's end the last residue stands in: no item reaches it).
-struct GeoR {
-  int base;
-  v3<double> p[4];
-  __device__ __forceinline__ v3<double> r(int i) const { return p[i - base]; }
-};
 
 // The static bonded terms of a system whose items are all chain-local. Each
 // thread takes one base residue per pass (consecutive residues on consecutive

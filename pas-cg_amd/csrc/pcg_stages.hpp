@@ -37,16 +37,14 @@ __device__ __forceinline__ void set_current_contact(const DevBatch &b, int q, in
                   ((uint32_t)((b.nc_i[1][c] - res0) & 0xFFF) << 12) | ((uint32_t)b.ncur_t[q] << 24);
 }
 
-__device__ inline int classify(const DevBatch &b, SysDescC &s, const SysState &st,
-                                        int slot) {
+// the lists of the NL pair (i1, i2) at distance d; native: it is a native contact
+__device__ inline int classify(const DevBatch &b, SysDescC &s, int i1, int i2, double d,
+                               bool native) {
   DevParamsC &P = *b.P;
   ParamsC &p = P.p;
-  int i1 = b.nl_i[0][slot], i2 = b.nl_i[1][slot];
-  double d = b.nl_d[slot];
-  double pad = st.orig_pad;
+  const double pad = p.nl_pad;
   bool four = b.chain[i1] == b.chain[i2] && abs(b.seq[i1] - b.seq[i2]) == 4;
-  if (p.nat_cont_on && s.nnc > 0 && d < __dadd_rn(p.nl_cutoff, pad) && find_contact(b, s, i1, i2) >= 0)
-    return CL_NC;
+  if (native && d < __dadd_rn(p.nl_cutoff, pad)) return CL_NC;
   if (p.qa_on && !(!p.qa_include4 && four) && d < __dadd_rn(p.nl_cutoff, pad))
     return CL_QA | (!(d > P.qa_max_req) ? CL_NEAR : 0);
   int cls = 0;
@@ -58,6 +56,30 @@ __device__ inline int classify(const DevBatch &b, SysDescC &s, const SysState &s
   if (P.pauli_on && d < __dadd_rn(p.rep_cutoff, pad)) cls |= CL_PAULI;
   return cls;
 }
+
+// Shares of one chain-local item: slot s receives the force on residue
+// base + s (s = 0..3), in registers.
+template <typename RF> struct AccSlots {
+  int base;
+  RF c[4][3];
+  template <typename T> __device__ __forceinline__ void add(int i, v3<T> f) {
+    int s = i - base;
+    // explicit selects keep c in registers
+    RF fx = (RF)f.x, fy = (RF)f.y, fz = (RF)f.z;
+    if (s == 0) { c[0][0] += fx; c[0][1] += fy; c[0][2] += fz; }
+    else if (s == 1) { c[1][0] += fx; c[1][1] += fy; c[1][2] += fz; }
+    else if (s == 2) { c[2][0] += fx; c[2][1] += fy; c[2][2] += fz; }
+    else { c[3][0] += fx; c[3][1] += fy; c[3][2] += fz; }
+  }
+};
+
+// The four residues of a base residue's items, read once for all of
+// them (past the chain's end the last residue stands in: no item reaches it).
+struct GeoR {
+  int base;
+  v3<double> p[4];
+  __device__ __forceinline__ v3<double> r(int i) const { return p[i - base]; }
+};
 
 // qa::finish_processing (cg/src/cg/qa/finish_processing.cpp:5-74), one block
 // per system: removals in contact order, candidates sorted by (distance,

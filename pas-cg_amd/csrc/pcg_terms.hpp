@@ -521,7 +521,7 @@ __device__ __forceinline__ bool pid_psi(const G &g, int i, int j, bool vp, bool 
 }
 
 template <typename R, typename G, typename A>
-__device__ double pid_item(const DevBatch &b, SysDescC &s, const G &g, A &acc, int k) {
+__device__ __forceinline__ double pid_item(const DevBatch &b, SysDescC &s, const G &g, A &acc, int k) {
   ParamsC &p = b.P->p;
   int i1 = b.pid_i[0][k], i2 = b.pid_i[1][k];
   if (b.atype[i1] == 14 || b.atype[i2] == 14) return 0.0; // PRO
