@@ -791,38 +791,224 @@ __global__ void k_prepare_nh(DevBatch b) {
   prepare_nh_item(b, g, i);
 }
 
-// The serial part of the finish (removals, then acceptance in order) reads
-// and writes the sync budgets of each candidate's residues: with
-// sync_lds the system's budgets sit in LDS for the kernel (one word a
-// residue, loaded and stored coalesced), and up to QF_CAND_LDS candidates
-// are staged there in acceptance order, so the serial loop waits on LDS
-// rather than on a chain of HBM loads.
-__global__ void k_qa_finish(DevBatch b, int sync_lds) {
+// Sums and differences of four int8 side by side, each on its own.
+__device__ __forceinline__ uint32_t add4(uint32_t x, uint32_t y) {
+  return ((x & 0x7f7f7f7fu) + (y & 0x7f7f7f7fu)) ^ ((x ^ y) & 0x80808080u);
+}
+__device__ __forceinline__ uint32_t sub4(uint32_t x, uint32_t y) {
+  return ((x | 0x80808080u) - (y & 0x7f7f7f7fu)) ^ ((x ^ ~y) & 0x80808080u);
+}
+// LDS of the QA finish beside the budgets: the candidates and the removed
+// contacts, as they come and in the order they are taken
+struct QfLds {
+  long long key[QF_CAND_LDS];   // by distance; then the accepted ones' ranks
+  uint64_t sd[QF_CAND_LDS];     // by rank: budget changes of the two residues,
+  int i1[QF_CAND_LDS], i2[QF_CAND_LDS], sc[QF_CAND_LDS];  // the residues, the slot
+  int idx[QF_CAND_LDS];
+  uint64_t rsd[QF_REM_LDS];     // by rank
+  int ri1[QF_REM_LDS], ri2[QF_REM_LDS];
+  int rem[QF_REM_LDS];          // as they come: 2 * contact + near
+  int wave[16];
+  int near, accepted, live, overflow;
+};
+
+// qa_finish_block (pcg_stages.hpp) by a whole workgroup of 1024, the budgets
+// in LDS (sy: one word of four a residue). Removed contacts and candidates are
+// ranked in parallel, one thread decides which candidates are taken, in order,
+// on LDS alone, and the lists are written and compressed in parallel. (With
+// that thread writing the lists too, a contact cost some 1 us of waits on HBM:
+// 18 us a step for the box of 6400 residues and 1240 us for its first, where
+// it is 8 and 316 so; what is left is the chain of loads and barriers.)
+__device__ __forceinline__ void qa_finish_wide(const DevBatch &b, SysDescC &sd, SysState &st,
+                                               uint32_t *sy, QfLds &q, int cand_n, int rem_n) {
+  const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wv = tid >> 6;
+  const int r0 = sd.res0, qc_n0 = st.qc_n, store0 = st.qf_store, qh0 = st.qh_n;
+  const int num0 = st.num_qa;
+  if (tid == 0) q.near = 0, q.overflow = 0;
+  for (int c = tid; c < cand_n; c += nt) {
+    q.key[c] = total_key(b.cand_dist[sd.nl0 + c]);
+    q.idx[c] = b.cand_idx[sd.nl0 + c];
+  }
+  for (int a = tid; a < rem_n; a += nt) {
+    const int v = b.rem[sd.qc0 + a];
+    q.rem[a] = 2 * v + (b.qc_d[sd.qc0 + v] > b.P->qa_max_req ? 0 : 1);
+  }
+  for (int k = tid; k < sd.n; k += nt) sy[k] = *(const uint32_t *)(b.sync + 4 * (r0 + k));
+  __syncthreads();
+  // candidates by (distance, free-pair index); ties, from evaluations repeated
+  // outside a step, as they came
+  for (int c = tid; c < cand_n; c += nt) {
+    const int sc = sd.nl0 + c, ic = q.idx[c];
+    const long long kc = q.key[c];
+    int rank = 0;
+    for (int o = 0; o < cand_n; ++o) {
+      const long long kd = q.key[o];
+      rank += (kd < kc || (kd == kc && (q.idx[o] < ic || (q.idx[o] == ic && o < c)))) ? 1 : 0;
+    }
+    q.sc[rank] = sc;
+    q.i1[rank] = b.cand_i[0][sc];
+    q.i2[rank] = b.cand_i[1][sc];
+    q.sd[rank] = *(const uint64_t *)(b.cand_sd + 8 * (size_t)sc);
+  }
+  // removed contacts in increasing index order, back among the free pairs
+  for (int a = tid; a < rem_n; a += nt) {
+    const int v = q.rem[a] >> 1, near = q.rem[a] & 1, qc = sd.qc0 + v;
+    int rank = 0, nearer = 0;
+    for (int o = 0; o < rem_n; ++o) {
+      const int w = q.rem[o];
+      const bool before = (w >> 1) < v || ((w >> 1) == v && o < a);
+      rank += before ? 1 : 0;
+      nearer += before ? (w & 1) : 0;
+    }
+    const int i1 = b.qc_i[0][qc], i2 = b.qc_i[1][qc];
+    q.ri1[rank] = i1 - r0;
+    q.ri2[rank] = i2 - r0;
+    q.rsd[rank] = *(const uint64_t *)(b.qc_sd + 8 * (size_t)qc);
+    b.qc_vac[qc] = 1;
+    const int slot = store0 + rank;
+    if (slot >= sd.qfcap) {
+      q.overflow = 1;
+      continue;
+    }
+    const int f = sd.qf0 + slot;
+    b.qf_i[0][f] = i1;
+    b.qf_i[1][f] = i2;
+    b.qf_d[f] = b.qc_d[qc];
+    b.qf_vac[f] = 0;
+    if (near) {
+      // appended at the end, so the near list stays in slot order
+      const int h = sd.qf0 + qh0 + nearer;
+      b.qh_slot[h] = slot;
+      b.qh_i[0][h] = i1;
+      b.qh_i[1][h] = i2;
+      b.qh_vac[h] = 0;
+      qa_near_filters(b, i1, i2, b.qh_req[h], b.qh_thr2[h]);
+      b.qh_ij[h] = (uint32_t)(i1 - r0) | ((uint32_t)(i2 - r0) << 16);
+      atomicAdd(&q.near, 1);
+    }
+  }
+  __syncthreads();
+  int *taken = (int *)q.key;
+  if (tid == 0) {
+    for (int a = 0; a < rem_n; ++a) {
+      const uint64_t v = q.rsd[a];
+      sy[q.ri1[a]] = add4(sy[q.ri1[a]], (uint32_t)v);
+      sy[q.ri2[a]] = add4(sy[q.ri2[a]], (uint32_t)(v >> 32));
+    }
+    int n = 0;
+    for (int a = 0; a < cand_n; ++a) {
+      const int i1 = q.i1[a] - r0, i2 = q.i2[a] - r0;
+      const uint64_t v = q.sd[a];
+      const uint32_t n1 = sub4(sy[i1], (uint32_t)v), n2 = sub4(sy[i2], (uint32_t)(v >> 32));
+      if ((n1 | n2) & 0x80808080u) continue;
+      if (qc_n0 + n >= sd.qccap) {
+        q.overflow = 1;
+        continue;
+      }
+      taken[n++] = a;
+      sy[i1] = n1;
+      sy[i2] = n2;
+    }
+    q.accepted = n;
+  }
+  __syncthreads();
+  for (int k = tid; k < sd.n; k += nt) *(uint32_t *)(b.sync + 4 * (r0 + k)) = sy[k];
+  const int acc_n = q.accepted;
+  for (int k = tid; k < acc_n; k += nt) {
+    const int a = taken[k], sc = q.sc[a], qc = sd.qc0 + qc_n0 + k;
+    b.qc_i[0][qc] = q.i1[a];
+    b.qc_i[1][qc] = q.i2[a];
+    b.qc_d[qc] = b.cand_od[sc];
+    b.qc_t[qc] = b.cand_t[sc];
+    b.qc_sat[qc] = 0.0;
+    *(uint64_t *)(b.qc_sd + 8 * (size_t)qc) = q.sd[a];
+    b.qc_vac[qc] = 0;
+    const int h = sd.qf0 + b.cand_h[sc];
+    b.qf_vac[sd.qf0 + b.cand_idx[sc]] = 1;
+    b.qh_vac[h] = 1;
+    b.qh_thr2[h] = -1.0f;
+  }
+  // compress: the contacts still there move to the front, in order, a block
+  // of them at a time (a contact never moves up, so no block's reads meet
+  // another's writes)
+  const int num = num0 - rem_n + acc_n;
+  int qc_n = qc_n0 + acc_n;
+  if (2 * num < qc_n) {
+    int slot = 0;
+    for (int base = 0; base < qc_n; base += nt) {
+      __syncthreads();
+      const int cur = base + tid, qc = sd.qc0 + cur;
+      const bool live = cur < qc_n && !b.qc_vac[qc];
+      const unsigned long long m = __ballot(live);
+      if (lane == 0) q.wave[wv] = __popcll(m);
+      int i1 = 0, i2 = 0;
+      double d = 0.0, sat = 0.0;
+      int16_t t = 0;
+      uint64_t v = 0;
+      if (live) {
+        i1 = b.qc_i[0][qc], i2 = b.qc_i[1][qc];
+        d = b.qc_d[qc], sat = b.qc_sat[qc];
+        t = b.qc_t[qc];
+        v = *(const uint64_t *)(b.qc_sd + 8 * (size_t)qc);
+      }
+      __syncthreads();
+      int at = slot + __popcll(m & ((1ull << lane) - 1ull));
+      for (int w = 0; w < nt >> 6; ++w) {
+        at += w < wv ? q.wave[w] : 0;
+        slot += q.wave[w];
+      }
+      if (live && at != cur) {
+        const int qs = sd.qc0 + at;
+        b.qc_i[0][qs] = i1;
+        b.qc_i[1][qs] = i2;
+        b.qc_d[qs] = d;
+        b.qc_t[qs] = t;
+        b.qc_sat[qs] = sat;
+        *(uint64_t *)(b.qc_sd + 8 * (size_t)qs) = v;
+        // the vacancy flag of the destination slot stays as it was
+      }
+    }
+    qc_n = slot;
+  }
+  if (tid == 0) {
+    const int back = min(rem_n, sd.qfcap - store0);
+    st.qf_n += back;
+    st.qf_store = store0 + back;
+    st.qh_n = qh0 + q.near;
+    st.num_qa = num;
+    st.qc_n = qc_n;
+    if (q.overflow) st.overflow = 1;
+    st.cand_n = 0;
+    st.rem_n = 0;
+  }
+}
+
+// The QA finish of a step, one workgroup a system: qa_finish_wide where the
+// budgets fit its LDS (sync_lds) and the candidates and removals their
+// staging, which only the first steps of a large system outgrow.
+__global__ __launch_bounds__(1024) void k_qa_finish(DevBatch b, int sync_lds) {
   extern __shared__ __align__(16) unsigned char qf_lds[];
   int s = blockIdx.x;
   SysState &st = b.st[s];
   if (!st.active || !b.P->p.qa_on) return;
   SysDescC &sd = b.sys[s];
+  // nothing removed and no candidate
+  if (st.cand_n == 0 && st.rem_n == 0) return;
+  const int rem_n = min(st.rem_n, sd.qccap), cand_n = min(st.cand_n, sd.nlcap);
   if (!sync_lds) {
     qa_finish_block(b, sd, st, b.sync, 0);
     return;
   }
-  // nothing removed and no candidate: the block's own early return, before
-  // any staging
-  if (st.cand_n == 0 && st.rem_n == 0) return;
   const int n = sd.n, r0 = sd.res0;
-  uint32_t *syl = (uint32_t *)qf_lds;
-  QfLds ql;
-  ql.key = (long long *)(qf_lds + 4 * (((size_t)sync_lds + 1) & ~(size_t)1));
-  ql.sd = (uint64_t *)(ql.key + QF_CAND_LDS);
-  ql.idx = (int *)(ql.sd + QF_CAND_LDS);
-  ql.sc = ql.idx + QF_CAND_LDS;
-  ql.i1 = ql.sc + QF_CAND_LDS;
-  ql.i2 = ql.i1 + QF_CAND_LDS;
-  ql.cap = QF_CAND_LDS;
+  QfLds &q = *(QfLds *)qf_lds;
+  uint32_t *syl = (uint32_t *)(qf_lds + sizeof(QfLds));
+  if (cand_n <= QF_CAND_LDS && rem_n <= QF_REM_LDS) {
+    qa_finish_wide(b, sd, st, syl, q, cand_n, rem_n);
+    return;
+  }
   for (int k = threadIdx.x; k < n; k += blockDim.x) syl[k] = *(const uint32_t *)(b.sync + 4 * (r0 + k));
   __syncthreads();
-  qa_finish_block(b, sd, st, (int8_t *)syl, r0, &ql);
+  qa_finish_block(b, sd, st, (int8_t *)syl, r0);
   for (int k = threadIdx.x; k < n; k += blockDim.x) *(uint32_t *)(b.sync + 4 * (r0 + k)) = syl[k];
 }
 
@@ -1360,7 +1546,7 @@ void launch_step_terms(const DevBatch &b, int prec, int max_n, bool step, hipStr
     hipLaunchKernelGGL(k_step_terms<float>, g, dim3(BLK), 0, s, b, step ? 1 : 0);
 }
 size_t qa_finish_lds(int max_n) {
-  return 4 * (((size_t)max_n + 1) & ~(size_t)1) + (size_t)QF_CAND_LDS * (8 + 8 + 4 * 4);
+  return sizeof(QfLds) + 4 * (((size_t)max_n + 1) & ~(size_t)1);
 }
 void launch_qa_finish(const DevBatch &b, int max_n, hipStream_t s) {
   // the budgets in LDS while they and the candidates fit 96 KB

@@ -11,9 +11,10 @@ constexpr int BLK = 256;
 // systems of this many residues or more take the NL row scan as a launch of
 // its own (k_nl_scan) instead of in the count pass's last row
 constexpr int ROWS_FUSE_MAX = 2048;
-// candidates the stage QA finish stages in LDS, and its LDS limit
-constexpr int QF_CAND_LDS = 1024;
-constexpr size_t QF_LDS_MAX = 96 * 1024;
+// candidates and removed contacts the stage QA finish stages in LDS, and its
+// LDS limit
+constexpr int QF_CAND_LDS = 2048, QF_REM_LDS = 512;
+constexpr size_t QF_LDS_MAX = 144 * 1024;
 
 // Geometry and per-residue QA data from HBM.
 struct GeoG {

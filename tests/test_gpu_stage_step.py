@@ -115,3 +115,24 @@ def test_forces_outside_a_step_are_the_arrays_forces():
     np.testing.assert_array_equal(c.get(6), f)
     np.testing.assert_array_equal(f, f.astype(np.float32))
     c.close()
+
+
+@pytest.mark.parametrize("copies,side,steps", [(1, 300.0, 20), (100, 150.0, 6), (100, 110.0, 6)])
+def test_qa_contacts_form_break_and_are_compressed(copies, side, steps):
+    # contacts that break within a few steps: in the first case the list is
+    # compressed on the way, in the others a step forms and breaks hundreds of
+    # contacts, in the last more than the finish stages in its LDS
+    over = {"qa_phase_dur": 0.02, "nat_cont_on": 0, "temperature": 3.0}
+    m = M.replicate(protein(41, 34), copies, side * A, 34)
+    o, c = Oracle(dict(FULL, **over), m, seed=3), stages(over, m)
+    o.set_noise_scale(0.0)
+    for _ in range(steps):
+        o.step(1)
+        c.step(1)
+        sync, num = c.qa_state()
+        assert num == o.num_qa_contacts()
+        np.testing.assert_array_equal(sync, o.sync())
+    ours, ref = c.list(6), o.list(6)
+    np.testing.assert_array_equal(np.stack(ours[:2]), np.stack(ref[:2]))
+    assert np.abs(c.get(0) - o.r()).max() < 1e-8
+    c.close()
