@@ -1348,9 +1348,10 @@ PersistentCfg persistent_cfg(DeviceBatch &B) {
 // per stage of the reference's step, optionally replayed as a hipGraph), or
 // the persistent kernel of the batched form for this one system (one
 // workgroup, many steps a launch, everything in LDS). The persistent form is
-// taken when the system fits its LDS, the noise is Philox (the reference's
+// possible when the system fits its LDS, the noise is Philox (the reference's
 // ran2 noise is drawn on the host every step) and there are no walls or box
-// protocol (which the stage path carries); a switch between the forms makes
+// protocol (which the stage path carries), and taken for all but large
+// systems (use_persistent); a switch between the forms makes
 // the next step rebuild the neighbour list, so that each form works on lists
 // it built itself.
 enum { FORM_NONE = 0, FORM_STAGES = 1, FORM_PERSISTENT = 2 };
@@ -1399,8 +1400,15 @@ bool persistent_eligible(const pcg_ctx &c) {
   const DeviceBatch &B = *c.B;
   return c.pcfg.ok && B.noise == PCG_NOISE_PHILOX && B.hp.p.n_walls == 0 && !B.box_set;
 }
+// PCG_FORM_AUTO: one workgroup's step grows with the system, the stages' is
+// their launches. us a step, persistent and stages, mixed precision: without
+// QA 500 residues 14 and 24, 700 18 and 24, 800 23 and 24, 900 26 and 24,
+// 1200 37 and 27; with QA 500 24 and 28, 600 31 and 29, 700 29 and 27, 900 42
+// and 28, 2000 148 and 36. The stages' forces are no less precise: they
+// accumulate in FP64 and take the bonded terms in FP64.
 bool use_persistent(const pcg_ctx &c) {
-  return c.form == PCG_FORM_PERSISTENT || (c.form == PCG_FORM_AUTO && persistent_eligible(c));
+  if (c.form != PCG_FORM_AUTO) return c.form == PCG_FORM_PERSISTENT;
+  return persistent_eligible(c) && c.B->max_n < (c.B->hp.p.qa_on ? 700 : 900);
 }
 // the first step in a form after steps in the other rebuilds the lists (the
 // device state records the form, so a restored checkpoint carries it)

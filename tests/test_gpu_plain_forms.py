@@ -79,3 +79,21 @@ def test_ineligible_contexts_keep_the_stages():
     c = G.Context(prm, m, precision=G.FP64, noise=G.PHILOX, seed=3)
     assert c.step_form(G.FORM_AUTO) == G.FORM_STAGES
     c.close()
+
+
+@pytest.mark.parametrize("qa_on,limit", [(1, 700), (0, 900)])
+def test_large_contexts_take_the_stages(qa_on, limit):
+    m = M.synthetic_protein(limit, M.job_seed(27))
+    prm = _prm(qa_on=qa_on)
+    auto = G.Context(prm, m, precision=G.FP64, noise=G.PHILOX, seed=11, philox_seed=5)
+    auto.set_noise_scale(0.0)
+    assert auto.step_form(G.FORM_AUTO) == G.FORM_STAGES
+    pers = _ctx(prm, m, G.FORM_PERSISTENT)
+    auto.step(40)
+    pers.step(40)
+    assert np.abs(auto.r() - pers.r()).max() < 1e-9
+    assert abs(auto.energy()[0] - pers.energy()[0]) <= 1e-9 * abs(auto.energy()[0])
+    auto.close()
+    pers.close()
+    small = M.synthetic_protein(limit - 1, M.job_seed(28))
+    _ctx(prm, small, G.FORM_AUTO).close()

@@ -117,7 +117,7 @@ def test_forces_outside_a_step_are_the_arrays_forces():
     c.close()
 
 
-@pytest.mark.parametrize("copies,side,steps", [(1, 300.0, 20), (100, 150.0, 6), (100, 110.0, 6)])
+@pytest.mark.parametrize("copies,side,steps", [(1, 300.0, 20), (100, 150.0, 6), (150, 170.0, 6)])
 def test_qa_contacts_form_break_and_are_compressed(copies, side, steps):
     # contacts that break within a few steps: in the first case the list is
     # compressed on the way, in the others a step forms and breaks hundreds of
