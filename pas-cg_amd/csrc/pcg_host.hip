@@ -1039,7 +1039,7 @@ int set_cols3(DeviceBatch &B, int s, double *const cols[3], const double *const 
 // system (cg/src/cg/langevin/step.cpp:119-127). The host draws a step's noise
 // into the next slot of the ring while the device runs the steps before; it
 // waits only for the kernel that read that slot NOISE_RING steps ago.
-int upload_ran2_noise(DeviceBatch &B) {
+int draw_ran2_noise(DeviceBatch &B, const double *&out) {
   const size_t ntot = B.d.ntot;
   if (!B.noise_pinned) {
     HIPCHK(hipHostMalloc((void **)&B.noise_pinned,
@@ -1055,7 +1055,12 @@ int upload_ran2_noise(DeviceBatch &B) {
     for (int c = 0; c < 3; ++c)
       for (int i = 0; i < d.n; ++i) nz[c * ntot + d.res0 + i] = B.ran2[s].normal();
   }
-  launch_noise_in(B.d, nz, B.stream);
+  out = nz;
+  return PCG_OK;
+}
+// after the launch that reads the last draw
+int ran2_noise_read(DeviceBatch &B) {
+  const int slot = (B.noise_at + DeviceBatch::NOISE_RING - 1) % DeviceBatch::NOISE_RING;
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(B.noise_read[slot], B.stream));
   return PCG_OK;
@@ -1375,7 +1380,8 @@ namespace {
 
 SysDesc *sys_rw(DeviceBatch &B) { return const_cast<SysDesc *>((const SysDesc *)B.d.sys); }
 
-void enqueue_step(DeviceBatch &B) {
+// noise: as launch_lang's
+void enqueue_step(DeviceBatch &B, const double *noise = nullptr) {
   const DevBatch &d = B.d;
   const pcg_params &p = B.hp.p;
   if (B.box_set) launch_box_phase(d, B.dP, sys_rw(B), B.stream);
@@ -1383,7 +1389,7 @@ void enqueue_step(DeviceBatch &B) {
   launch_step_terms(d, B.prec, B.max_n, true, B.stream);
   if (p.qa_on) launch_qa_finish(d, B.max_n, B.stream);
   if (B.hp.ljw_terms) launch_ljw_process(d, B.stream);
-  launch_lang(d, B.prec, B.noise, B.stream, true, B.box_set);
+  launch_lang(d, B.prec, B.noise, noise, B.stream, true, B.box_set);
 }
 
 // the host copy of the system descriptor after the box protocol moved the
@@ -1514,8 +1520,15 @@ int pcg_step(pcg_ctx *c, int32_t nsteps) {
   }
   if ((rc = switch_form(*c, FORM_STAGES))) return rc;
   for (int k = 0; k < nsteps; ++k) {
-    if (B.noise == PCG_NOISE_RAN2 && (rc = upload_ran2_noise(B))) return rc;
+    const bool ran2 = B.noise == PCG_NOISE_RAN2;
+    const double *noise = nullptr;
+    if (ran2 && (rc = draw_ran2_noise(B, noise))) return rc;
     if (c->graph_on) {
+      // a replayed step reads its noise at one address, on the device
+      if (ran2) {
+        launch_noise_in(B.d, noise, B.stream);
+        if ((rc = ran2_noise_read(B))) return rc;
+      }
       if (!c->gexec) {
         HIPCHK(hipStreamBeginCapture(B.stream, hipStreamCaptureModeThreadLocal));
         enqueue_step(B);
@@ -1524,7 +1537,8 @@ int pcg_step(pcg_ctx *c, int32_t nsteps) {
       }
       HIPCHK(hipGraphLaunch(c->gexec, B.stream));
     } else {
-      enqueue_step(B);
+      enqueue_step(B, noise);
+      if (ran2 && (rc = ran2_noise_read(B))) return rc;
     }
   }
   HIPCHK(hipStreamSynchronize(B.stream));
@@ -1699,11 +1713,13 @@ int pcg_lang_step(pcg_ctx *c) {
   DeviceBatch &B = *c->B;
   int rc = switch_form(*c, FORM_STAGES);
   if (rc) return rc;
-  if (B.noise == PCG_NOISE_RAN2 && (rc = upload_ran2_noise(B))) return rc;
+  const double *noise = nullptr;
+  if (B.noise == PCG_NOISE_RAN2 && (rc = draw_ran2_noise(B, noise))) return rc;
   // the forces it takes are those a caller sees: an evaluation's, a step's or
   // a restored state's
   if (B.prec != PCG_FP64) launch_load_forces(B.d, B.stream);
-  launch_lang(B.d, B.prec, B.noise, B.stream);
+  launch_lang(B.d, B.prec, B.noise, noise, B.stream);
+  if (noise && (rc = ran2_noise_read(B))) return rc;
   launch_tick(B.d, 1, B.stream);
   HIPCHK(hipStreamSynchronize(B.stream));
   return PCG_OK;

@@ -1096,25 +1096,27 @@ __global__ void k_tick(DevBatch b, int advance, int nl_done) {
 // read before the count, as it is final by then. log (one system): one more
 // block than the residues need keeps the wall forces' log, which reads the
 // time too, and counts itself as one more item.
-template <typename RF> __global__ void k_lang(DevBatch b, int noise_mode, int tick, int log) {
+//
+// noise (RAN2): the step's draws where the host put them (ntot x, then y, then
+// z), or null for the device's copy. Read from host memory here, they cost a
+// step 1.1 us; a kernel that copied them took 4.8.
+template <typename RF>
+__global__ void k_lang(DevBatch b, int noise_mode, const double *noise, int tick, int log) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   int s = -1, sys = -1;
   bool mine = false;   // a residue of an active system
   double disp = -1.0;  // below every displacement: lanes without a residue
   if (i < b.ntot) {
+    // (the longest wait first)
+    double nz[3];
+    if (noise_mode == PCG_NOISE_RAN2)
+      for (int c = 0; c < 3; ++c) nz[c] = noise ? noise[(size_t)c * b.ntot + i] : b.noise[c][i];
     s = sys = b.sysid[i];
     SysState &st = b.st[s];
     mine = st.active != 0;
     if (st.active && b.P->p.lang_on) {
       SysDescC &sd = b.sys[s];
-      double nz[3];
-      if (noise_mode == PCG_NOISE_RAN2) {
-        nz[0] = b.noise[0][i];
-        nz[1] = b.noise[1][i];
-        nz[2] = b.noise[2][i];
-      } else {
-        philox_normals(sd.philox_key, st.step, b.local[i], nz);
-      }
+      if (noise_mode != PCG_NOISE_RAN2) philox_normals(sd.philox_key, st.step, b.local[i], nz);
       const double F[3] = {b.acc[0][i], b.acc[1][i], b.acc[2][i]};
       double r[3];
       gear_update(b, sd, st, i, F[0], F[1], F[2], nz, r);
@@ -1554,14 +1556,15 @@ void launch_qa_finish(const DevBatch &b, int max_n, hipStream_t s) {
   const int sync_lds = lds <= QF_LDS_MAX ? max_n : 0;
   hipLaunchKernelGGL(k_qa_finish, dim3(b.nsys), dim3(1024), sync_lds ? lds : 0, s, b, sync_lds);
 }
-void launch_lang(const DevBatch &b, int prec, int noise_mode, hipStream_t s, bool tick, bool log) {
+void launch_lang(const DevBatch &b, int prec, int noise_mode, const double *noise,
+                 hipStream_t s, bool tick, bool log) {
   const int t = tick ? 1 : 0, l = log ? 1 : 0;
   dim3 g = grid1(b.ntot);
   g.x += l;
   if (prec == PCG_FP64)
-    hipLaunchKernelGGL(k_lang<double>, g, dim3(BLK), 0, s, b, noise_mode, t, l);
+    hipLaunchKernelGGL(k_lang<double>, g, dim3(BLK), 0, s, b, noise_mode, noise, t, l);
   else
-    hipLaunchKernelGGL(k_lang<float>, g, dim3(BLK), 0, s, b, noise_mode, t, l);
+    hipLaunchKernelGGL(k_lang<float>, g, dim3(BLK), 0, s, b, noise_mode, noise, t, l);
 }
 void launch_tick(const DevBatch &b, int advance, hipStream_t s, bool nl_done) {
   hipLaunchKernelGGL(k_tick, grid1(b.nsys, 64), dim3(64), 0, s, b, advance, nl_done ? 1 : 0);

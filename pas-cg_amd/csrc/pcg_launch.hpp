@@ -46,8 +46,9 @@ void launch_terms(const DevBatch &b, int prec, int max_items, int term, int from
 void launch_qa_finish(const DevBatch &b, int max_n, hipStream_t s);
 // tick: the step's k_tick (advance, close a rebuild) by the wave that
 // completes each system, log: after the wall forces' log of the box protocol
-void launch_lang(const DevBatch &b, int prec, int noise_mode, hipStream_t s, bool tick = false,
-                 bool log = false);
+// noise: RAN2 draws in host memory, or null for those on the device
+void launch_lang(const DevBatch &b, int prec, int noise_mode, const double *noise, hipStream_t s,
+                 bool tick = false, bool log = false);
 void launch_tick(const DevBatch &b, int advance, hipStream_t s, bool nl_done = false);
 // walls and the box protocol of a plain context (b.wall set): LJ candidate
 // processing; box set-up, and the phase logic before a step. P and sd are the
