@@ -114,8 +114,12 @@ __global__ __launch_bounds__(1024) void k_fetch(const uint32_t *words, uint32_t 
     if (acc) ((T *)col)[k] = (T)acc[(size_t)c * n + k];
     out[i] = (double)col[k];
   }
+  // The stores go to host memory and a barrier waits for none of them: each
+  // wave releases its own to the system first. Without a flag too, as the
+  // flagged fetch behind this one on the stream may run on another XCD, whose
+  // release covers its own L2 only.
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
   if (!flag) return;
-  // every wave's stores are out before the barrier; one release covers them
   __syncthreads();
   if (threadIdx.x == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
