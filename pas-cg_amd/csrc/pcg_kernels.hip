@@ -114,14 +114,19 @@ __global__ __launch_bounds__(1024) void k_fetch(const uint32_t *words, uint32_t 
     if (acc) ((T *)col)[k] = (T)acc[(size_t)c * n + k];
     out[i] = (double)col[k];
   }
-  // The stores go to host memory and a barrier waits for none of them: each
-  // wave releases its own to the system first. Without a flag too, as the
-  // flagged fetch behind this one on the stream may run on another XCD, whose
-  // release covers its own L2 only.
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
-  if (!flag) return;
+  // A barrier waits for no store, and thread 0's release for its own wave's
+  // only. So every wave waits until its stores are in the L2, which is the
+  // workgroup's waves' own and which thread 0 then writes back to the system:
+  // also without a flag, as the flagged fetch behind on the stream may run on
+  // another XCD. (A system release by every wave does it too, but 16
+  // write-backs of the L2 took 5 us more a call.)
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   __syncthreads();
-  if (threadIdx.x == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+    if (flag) __hip_atomic_store(flag, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 // the host's noise for one step (ntot x, then y, then z) into the device's
 __global__ void k_noise_in(DevBatch b, const double *src) {
