@@ -941,8 +941,18 @@ int make_batch(const pcg_params &p, int nsys, const pcg_model *models, const dou
 // Enqueues a fetch into the batch's pinned memory (its room already made) and
 // waits for it to arrive: the host reads the flag for a while, which a fetch
 // behind idle work raises within some microseconds, then waits for the stream.
+// From 15 000 values on (5000 residues) many workgroups and a wait for the
+// stream: one workgroup writes some 10 GB/s to the host. us a call for a
+// system's positions, one workgroup and many: 2000 residues 13 and 16, 4000
+// 17 and 18, 6400 22 and 21, 25 600 64 and 41, 102 400 256 and 175.
 int fetch_now(DeviceBatch &B, Fetch f) {
   Pinned &pin = *B.pin;
+  if (std::max(f.bytes / 4, (size_t)3 * f.n) >= 15000) {
+    launch_fetch(f, B.stream);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(B.stream));
+    return PCG_OK;
+  }
   f.flag = pin.flag;
   f.seq = ++pin.seq;
   launch_fetch(f, B.stream);
@@ -997,9 +1007,6 @@ int get_cols(DeviceBatch &B, int s, double *const cols[3], double *out) {
   const void *c[3] = {cols[0], cols[1], cols[2]};
   return get_triples(B, s, c, false, out);
 }
-int get_forces(DeviceBatch &B, int s, double *out) {
-  return get_triples(B, s, B.d.F, B.prec != PCG_FP64, out);
-}
 
 // The same three columns to or from caller arrays of one component each,
 // element i at comp[c][i * stride].
@@ -1007,10 +1014,52 @@ void spread3(const double *triples, int n, double *const out[3], int64_t stride)
   for (int i = 0; i < n; ++i)
     for (int c = 0; c < 3; ++c) out[c][(size_t)i * stride] = triples[3 * (size_t)i + c];
 }
+// From this many residues on, columns that the triples of a fetch would only
+// detour come as copies: FP64 columns into component arrays without one more
+// pass on the host, FP32 columns at half the bytes. us a call, copies and
+// fetch: component arrays of 25 600 residues 58 and 56, of 102 400 150 and
+// 182; FP32 forces 51 and 41, 135 and 172.
+constexpr int COPY_COLS_MIN = 32768;
+int copy_cols(DeviceBatch &B, int s, const void *const cols[3], size_t esz, void *const out[3]) {
+  const size_t n = B.sys[s].n, r0 = B.sys[s].res0;
+  for (int c = 0; c < 3; ++c)
+    HIPCHK(hipMemcpyAsync(out[c], (const char *)cols[c] + esz * r0, esz * n, hipMemcpyDeviceToHost,
+                          B.stream));
+  HIPCHK(hipStreamSynchronize(B.stream));
+  return PCG_OK;
+}
+template <typename T>
+int copy_cols3(DeviceBatch &B, int s, const void *const cols[3], double *const out[3],
+               int64_t stride) {
+  const size_t n = B.sys[s].n;
+  if (stride == 1 && sizeof(T) == 8) {
+    void *const to[3] = {out[0], out[1], out[2]};
+    return copy_cols(B, s, cols, 8, to);
+  }
+  std::vector<T> tmp(3 * n);
+  void *const to[3] = {tmp.data(), tmp.data() + n, tmp.data() + 2 * n};
+  const int rc = copy_cols(B, s, cols, sizeof(T), to);
+  if (rc) return rc;
+  const bool triples = stride == 3 && out[1] == out[0] + 1 && out[2] == out[0] + 2;
+  double *const o = out[0];
+  for (size_t i = 0; i < n; ++i)
+    for (int c = 0; c < 3; ++c)
+      (triples ? o[3 * i + c] : out[c][i * stride]) = (double)tmp[c * n + i];
+  return PCG_OK;
+}
+int get_forces(DeviceBatch &B, int s, double *out) {
+  const bool f32 = B.prec != PCG_FP64;
+  if (!f32 || B.sys[s].n < COPY_COLS_MIN) return get_triples(B, s, B.d.F, f32, out);
+  double *const comp[3] = {out, out + 1, out + 2};
+  return copy_cols3<float>(B, s, B.d.F, comp, 3);
+}
 int get_cols3(DeviceBatch &B, int s, const void *const cols[3], bool f32, double *const out[3],
               int64_t stride) {
   const int n = B.sys[s].n;
   HIPCHK(hipSetDevice(B.device));
+  if (n >= COPY_COLS_MIN)
+    return f32 ? copy_cols3<float>(B, s, cols, out, stride)
+               : copy_cols3<double>(B, s, cols, out, stride);
   int rc = B.pin->room(24 * (size_t)n);
   if (rc || (rc = fetch_now(B, fetch_of(B, s, cols, f32, 0)))) return rc;
   spread3((const double *)B.pin->p, n, out, stride);

@@ -98,17 +98,19 @@ __global__ void k_mark_invalid(DevBatch b) {
 }
 
 // Device data into mapped pinned host memory: words as they are, and three
-// columns as interleaved FP64 triples; one workgroup, which then writes seq to
-// the host's flag, so that the host sees the result arrive by reading the flag
+// columns as interleaved FP64 triples. One workgroup then writes seq to the
+// host's flag, so that the host sees the result arrive by reading the flag
 // instead of waiting for the stream (9 us a call for a system's positions;
 // 14 us with a wait for the stream, 47 us as three staged column copies).
+// Without a flag, any number of workgroups.
 template <typename T>
 __global__ __launch_bounds__(1024) void k_fetch(const uint32_t *words, uint32_t *words_out, int nw,
                                                 const T *x, const T *y, const T *z,
                                                 const double *acc, double *out, int n, int *flag,
                                                 int seq) {
-  for (int i = threadIdx.x; i < nw; i += blockDim.x) words_out[i] = words[i];
-  for (int i = threadIdx.x; i < 3 * n; i += blockDim.x) {
+  const int i0 = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+  for (int i = i0; i < nw; i += stride) words_out[i] = words[i];
+  for (int i = i0; i < 3 * n; i += stride) {
     const int k = i / 3, c = i - 3 * k;
     const T *col = c == 0 ? x : c == 1 ? y : z;
     if (acc) ((T *)col)[k] = (T)acc[(size_t)c * n + k];
@@ -1498,13 +1500,14 @@ void launch_mark_invalid(const DevBatch &b, hipStream_t s) {
 void launch_fetch(const Fetch &f, hipStream_t s) {
   const int most = std::max((int)(f.bytes / 4), 3 * f.n);
   const dim3 block((unsigned)std::min(1024, std::max(64, (most + 63) / 64 * 64)));
+  const dim3 grid(f.flag ? 1u : (unsigned)std::min(64, std::max(1, (most + 1023) / 1024)));
   if (f.f32)
-    hipLaunchKernelGGL(k_fetch<float>, dim3(1), block, 0, s, (const uint32_t *)f.src,
+    hipLaunchKernelGGL(k_fetch<float>, grid, block, 0, s, (const uint32_t *)f.src,
                        (uint32_t *)f.dst, (int)(f.bytes / 4), (const float *)f.cols[0],
                        (const float *)f.cols[1], (const float *)f.cols[2], f.acc, f.out, f.n, f.flag,
                        f.seq);
   else
-    hipLaunchKernelGGL(k_fetch<double>, dim3(1), block, 0, s, (const uint32_t *)f.src,
+    hipLaunchKernelGGL(k_fetch<double>, grid, block, 0, s, (const uint32_t *)f.src,
                        (uint32_t *)f.dst, (int)(f.bytes / 4), (const double *)f.cols[0],
                        (const double *)f.cols[1], (const double *)f.cols[2], (const double *)nullptr, f.out, f.n,
                        f.flag, f.seq);

@@ -82,3 +82,38 @@ def test_overflow_is_reported_and_stays():
     with pytest.raises(G.PcgError):
         c.step(0)
     c.close()
+
+
+@pytest.mark.parametrize("n", [4999, 5000, 32767, 32768])
+@pytest.mark.parametrize("precision", [G.FP64, G.MIXED], ids=["fp64", "mixed"])
+def test_large_results(n, precision):
+    """Sizes on both sides of the lines between the fetch's forms: what is set
+    comes back bit for bit, and the forces of one tethered pair in the last
+    residues only there."""
+    p = W.base_params()
+    side = int(np.ceil(n ** (1 / 3)))
+    pos = np.stack(np.unravel_index(np.arange(n), (side,) * 3), axis=1) * 8.0
+    pos[n - 1] = pos[n - 2] + [0.0, 0.0, 0.9]
+    m = {"n": n, "pos": pos, "orig_pos": pos * 0.5, "atype": np.zeros(n, np.uint8),
+         "chain": np.zeros(n, np.int32), "seq": np.arange(n, dtype=np.int32), "cell": np.zeros(3),
+         "teth": np.array([[n - 2, n - 1]], np.int32), "ang": np.zeros((0, 3), np.int32),
+         "dih": np.zeros((0, 4), np.int32), "cont": np.zeros((0, 2), np.int32),
+         "ang_has": np.zeros(0, np.uint8), "dih_has": np.zeros(0, np.uint8),
+         "ang_theta": np.zeros(0), "dih_phi": np.zeros(0), "cont_len": np.zeros(0),
+         "cont_type": np.zeros(0, np.int32)}
+    c = G.Context(p, M.empty_tips(m), precision=precision, seed=1)
+    rng = np.random.default_rng(n)
+    for which in (1, 5):
+        x = rng.normal(size=(n, 3))
+        c.set(which, x)
+        np.testing.assert_array_equal(c.get(which), x)
+        np.testing.assert_array_equal(c.get3(which).T, x)
+    c.eval_term("tether")
+    F = c.get(6)
+    np.testing.assert_array_equal(F, c.get3(6).T)
+    assert not F[:n - 2].any()
+    dr = 0.9 - 0.45
+    want = min(dr * (p["tether_H1"] + 2 * p["tether_H2"] * dr * dr), 1e3)  # the harmonic's limit
+    np.testing.assert_allclose(F[n - 2:, 2], [want, -want], rtol=1e-6)
+    np.testing.assert_array_equal(F, c.eval_term3("tether")[0].T)
+    c.close()
