@@ -187,8 +187,10 @@ __device__ __forceinline__ unsigned long long lane_u64(unsigned long long v, int
 // coordinate staged, d the threshold): staging rounds a coordinate by at most
 // 2^-24 M and the difference, squares and sums round by at most a few 2^-24,
 // together less than 4.2e-7 M / d + 4e-7. Pairs inside a margin are kept and
-// counted by the classification. In a periodic cell the differences are
-// formed and wrapped in FP64 and rounded afterwards (M = 0).
+// counted by the classification. In a periodic cell, and in a system with a
+// coordinate beyond 1e4 NL radii or none at all (a diverged one: up to there
+// the margin is a hundredth, an infinite one would keep every column), the
+// differences are formed (and wrapped) in FP64 and rounded afterwards (M = 0).
 //
 // QA free pairs beyond the QA maximum required distance are counted (qf_n,
 // which sizes the contact loop as the reference's free-pair count does) but
@@ -228,9 +230,10 @@ __device__ __forceinline__ void wg_fix_nl(DevBatchC *bp, int s, SysState &st, co
   __shared__ int wirr[16];
   __shared__ u64 charge_mask[64];  // the charged residues of each 64
   const bool cell = has_cell(sd);
+  const float far_from = 1e4f * (float)(P.nl_eff_cutoff + p.nl_pad);
   const double ox = g.x[0], oy = g.y[0], oz = g.z[0];
   float span = 0.0f;
-  bool irr = false;
+  bool irr = false, far = false;
   for (int k0 = threadIdx.x - lane; k0 < n; k0 += blockDim.x) {
     const int k = k0 + lane;
     const u64 cm = __ballot(k < n && ((chg >> (g.at[min(k, n - 1)] & 31)) & 1u));
@@ -251,10 +254,11 @@ __device__ __forceinline__ void wg_fix_nl(DevBatchC *bp, int s, SysState &st, co
     }
     const float fx = (float)(g.x[k] - ox), fy = (float)(g.y[k] - oy), fz = (float)(g.z[k] - oz);
     span = fmaxf(span, fmaxf(fabsf(fx), fmaxf(fabsf(fy), fabsf(fz))));
+    far |= !(fabsf(fx) <= far_from) | !(fabsf(fy) <= far_from) | !(fabsf(fz) <= far_from);
     pos4[k] = make_float4(fx, fy, fz, __builtin_bit_cast(float, (uint32_t)(g.at[k] & 31) | (mate << 8)));
   }
   for (int o = 32; o > 0; o >>= 1) span = fmaxf(span, __shfl_down(span, o, 64));
-  const bool wave_irr = __any(irr);
+  const int wave_irr = (__any(irr) ? 1 : 0) | (__any(far) ? 2 : 0);
   if (lane == 0) {
     wspan[w] = span;
     wirr[w] = wave_irr;
@@ -284,13 +288,14 @@ __device__ __forceinline__ void wg_fix_nl(DevBatchC *bp, int s, SysState &st, co
   const bool qa_on = p.qa_on, pid_on = p.pid_on, dh_on = p.dh_on, pauli_on = P.pauli_on;
   const bool qa4 = p.qa_include4, pid4 = p.pid_include4;
   __syncthreads();
-  bool regular = true;
+  int all_irr = 0;
   span = 0.0f;
   for (int v = 0; v < nw; ++v) {
     span = fmaxf(span, wspan[v]);
-    regular = regular && !wirr[v];
+    all_irr |= wirr[v];
   }
-  if (cell) span = 0.0f;
+  const bool regular = !(all_irr & 1), by64 = cell | ((all_irr & 2) != 0);
+  if (by64) span = 0.0f;
   // squared thresholds in FP32, their margins (half) in the FP32 comparisons,
   // and the bounds clear of them; in scalar registers
   auto half = [&](double t) {
@@ -347,7 +352,7 @@ __device__ __forceinline__ void wg_fix_nl(DevBatchC *bp, int s, SysState &st, co
   // a pair's squared distance as the scan sees it
   auto scan_d2 = [&](float4 q, float xi, float yi, float zi, int k, int j) {
     float dx = q.x - xi, dy = q.y - yi, dz = q.z - zi;
-    if (cell) {
+    if (by64) {
       const v3<double> dd = xwrapd(xsub(v3<double>{g.x[j], g.y[j], g.z[j]},
                                         v3<double>{g.x[k], g.y[k], g.z[k]}), sd);
       dx = (float)dd.x, dy = (float)dd.y, dz = (float)dd.z;
@@ -358,7 +363,7 @@ __device__ __forceinline__ void wg_fix_nl(DevBatchC *bp, int s, SysState &st, co
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m, base));
   };
-  const bool plain = regular && !cell && !keep4;
+  const bool plain = regular && !by64 && !keep4;
   int kept = 0;
   u64 native_in = 0ull;
   for (int pass = 0; pass < 2; ++pass) {
@@ -395,7 +400,8 @@ __device__ __forceinline__ void wg_fix_nl(DevBatchC *bp, int s, SysState &st, co
                 if (jc == W - 1) cols &= last_cols;
                 const float dx = q.x - xi, dy = q.y - yi, dz = q.z - zi;
                 float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-                d2 = __builtin_amdgcn_inverse_ballot_w64(cols) ? d2 : 1e30f;
+                // (no comparison takes a NaN, whatever the thresholds)
+                d2 = __builtin_amdgcn_inverse_ballot_w64(cols) ? d2 : __builtin_nanf("");
                 lane_in += d2 < nl_lo ? 1 : 0;
                 lane_inner += d2 < nc_lo ? 1 : 0;
                 // one test for all reasons to keep a pair: inside keep_to, or

@@ -52,6 +52,14 @@ def in_cell(n):
     return m
 
 
+def far_off(n, k, x):
+    """Residue k far outside, as a diverged trajectory leaves it."""
+    m = protein(n)
+    m["pos"] = m["pos"].copy()
+    m["pos"][k] = x
+    return m
+
+
 FULL = W.full_params()
 NO_QA = dict(FULL, qa_on=0, pid_on=1)
 GO = W.base_params()
@@ -66,6 +74,9 @@ CASES += [("four", FOUR, protein(150)), ("four-dh", FOUR_DH, protein(150)),
           ("swapped", NO_QA, two_chains(150, swap=True)), ("arc", FULL, stretched(200)),
           ("arc-noqa", NO_QA, stretched(200)), ("cell", FULL, in_cell(150)),
           ("cell-four", FOUR, in_cell(150)), ("long", FULL, protein(900))]
+CASES += [(f"off-{k}-{x:g}", FULL, far_off(150, k, x)) for k in (0, 77) for x in (1e5, 1e20, 1e200, np.inf)]
+CASES += [("off-noqa", NO_QA, far_off(150, 149, [1e40, 0.0, 0.0])),
+          ("reach", dict(FULL, nl_cutoff=1e16, dh_cutoff=1e16), protein(40))]
 
 
 @pytest.mark.parametrize("prm,m", [c[1:] for c in CASES], ids=[c[0] for c in CASES])
@@ -97,3 +108,19 @@ def test_lists_equal_the_oracles(prm, m):
     b.run(1)
     assert b.sizes(0)["nl"] == len(o.list(0)[0])
     b.close()
+
+
+def test_a_diverged_system_stays_alone():
+    """Systems of a batch beside ones with coordinates FP32 cannot hold."""
+    ms = [protein(100, 1), far_off(100, 7, np.inf), protein(130, 2), far_off(64, 0, 1e300), protein(90, 3)]
+    # the same places (and so the same noise) with ordinary systems between
+    calm = [protein(m["n"], 9) if k % 2 else m for k, m in enumerate(ms)]
+    b, o = (G.Batch(FULL, x, seeds=[1, 2, 3, 4, 5], precision=G.MIXED) for x in (ms, calm))
+    b.run(3)
+    o.run(3)
+    for k in (0, 2, 4):
+        assert b.sizes(k) == o.sizes(k)
+        # three steps of mixed forces summed in another order
+        np.testing.assert_allclose(b.get(k, 0), o.get(k, 0), rtol=0, atol=1e-9)
+    b.close()
+    o.close()
