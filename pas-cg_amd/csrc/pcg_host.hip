@@ -1466,7 +1466,8 @@ bool use_persistent(const pcg_ctx &c) {
   return persistent_eligible(c) && c.B->max_n < (c.B->hp.p.qa_on ? 700 : 900);
 }
 // the first step in a form after steps in the other rebuilds the lists (the
-// device state records the form, so a restored checkpoint carries it)
+// device state records the form, so a restored checkpoint carries it); calls
+// term by term before it work on the persistent kernel's lists
 int switch_form(pcg_ctx &c, int to) {
   DeviceBatch &B = *c.B;
   if (c.last_form == to) return PCG_OK;
@@ -1477,8 +1478,13 @@ int switch_form(pcg_ctx &c, int to) {
     st.verify_first = 1;
     st.nl_invalid = 1;
   }
+  const bool near_fields = st.form == FORM_PERSISTENT && B.hp.p.qa_on;
   st.form = to;
   if ((rc = write_state(B, 0, st))) return rc;
+  if (near_fields) {
+    launch_near_fields(B.d, B.stream);
+    HIPCHK(hipGetLastError());
+  }
   c.last_form = to;
   return PCG_OK;
 }

@@ -11,6 +11,8 @@ void launch_eval_begin(const DevBatch &b, hipStream_t s);
 void launch_store_forces(const DevBatch &b, hipStream_t s);
 // and back
 void launch_load_forces(const DevBatch &b, hipStream_t s);
+// completes near lists of the persistent kernel for the stage kernels
+void launch_near_fields(const DevBatch &b, hipStream_t s);
 void launch_mark_invalid(const DevBatch &b, hipStream_t s);
 // device data into mapped pinned host memory: bytes of src as words, and three
 // columns of n values (FP32 or FP64) as FP64 triples; then seq into flag. acc

@@ -7,9 +7,11 @@ keep the stage form."""
 import numpy as np
 import pytest
 
+from oracle_ffi import Oracle
 from pas_cg_amd import model as M
 from pas_cg_amd import params as P
 from pas_cg_amd import pcg as G
+from pas_cg_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
 
@@ -97,3 +99,56 @@ def test_large_contexts_take_the_stages(qa_on, limit):
     pers.close()
     small = M.synthetic_protein(limit - 1, M.job_seed(28))
     _ctx(prm, small, G.FORM_AUTO).close()
+
+
+@pytest.mark.parametrize("stage_step", [False, True], ids=["fresh", "after stages"])
+@pytest.mark.parametrize("qa_on", [1, 0], ids=["qa", "no qa"])
+@pytest.mark.parametrize("prec,eF,eV", [(G.FP64, 1e-9, 1e-9), (G.MIXED, 1e-5, 1e-6)],
+                         ids=["fp64", "mixed"])
+def test_per_term_calls_on_the_persistent_lists(prec, eF, eV, qa_on, stage_step):
+    """The terms one by one and together, on the lists the persistent kernel
+    left, in a context that never built any in the stage form and in one whose
+    stage lists are of other positions."""
+    prm = dict(W.full_params(), qa_on=qa_on)
+    m = M.synthetic_protein(150, M.job_seed(29), heuristic_frac=0.3)
+    rng = np.random.default_rng(29)
+    m["pos"] = m["pos"] + rng.normal(scale=0.2 * P.ANGSTROM, size=(150, 3))
+    o = Oracle(prm, m, seed=4)
+    c = G.Context(prm, m, precision=prec, noise=G.PHILOX, seed=4)
+    o.set_noise_scale(0.0)
+    c.set_noise_scale(0.0)
+    if stage_step:
+        c.step_form(G.FORM_STAGES)
+        o.step(1)
+        c.step(1)
+        r = o.r()
+        r = r[::-1] + rng.normal(scale=0.1 * P.ANGSTROM, size=r.shape)  # other pairs are near
+        o.set_r(r)
+        c.set(0, r)
+        o.fix_nl()
+    c.step_form(G.FORM_PERSISTENT)
+    o.step(1)
+    c.step(1)
+    # (both on the same positions: mixed steps round)
+    c.set(0, o.r())
+    o.prepare_nh()
+    c.prepare_nh()
+    for term, on in W.term_enabled(prm).items():
+        if not on:
+            continue
+        F, V = c.eval_term(term)
+        Fo, Vo = o.eval_term(term)
+        err = float(np.abs(F - Fo).max())
+        assert err <= eF * max(float(np.abs(Fo).max()), 1e-12), term
+        assert abs(V - Vo) <= eV * max(abs(Vo), 1e-12), term
+    c.eval_forces()
+    o.eval_forces()
+    err = float(np.abs(c.get(6) - o.F()).max())
+    assert err <= eF * float(np.abs(o.F()).max())
+    if qa_on:
+        c.qa_finish()
+        o.qa_finish()
+        sync, num = c.qa_state()
+        assert num == o.num_qa_contacts()
+        np.testing.assert_array_equal(sync, o.sync())
+    c.close()
