@@ -1157,6 +1157,9 @@ __global__ void k_lang(DevBatch b, int noise_mode, const double *noise, int tick
       disp = disp_from_orig(b, sd, i, r);
     } else {
       s = -1;
+      // without Langevin steps the forces are a step's result all the same
+      if (sizeof(RF) == 4 && mine)
+        for (int c = 0; c < 3; ++c) ((RF *)b.F[c])[i] = (RF)b.acc[c][i];
     }
   } else if (log && blockIdx.x == gridDim.x - 1 && threadIdx.x < 7) {
     mine = threadIdx.x == 0 && b.st[0].active != 0;

@@ -102,6 +102,33 @@ def test_a_batch_of_stage_systems():
     b.close()
 
 
+@pytest.mark.parametrize("prec,tol", [(G.FP64, 1e-9), (G.MIXED, 1e-5)], ids=["fp64", "mixed"])
+def test_forces_of_steps_without_langevin(prec, tol):
+    """A step that does not integrate leaves its forces where they are read, of
+    a plain context, of a batch on the stage kernels, and in a saved state."""
+    p = dict(FULL, lang_on=0)
+    m = protein(130)
+    o = Oracle(p, m, seed=3)
+    o.step(1)
+    F = o.F()
+    c = stages({"lang_on": 0}, m, prec)
+    c.step(1)
+    err = float(np.abs(c.get(6) - F).max())
+    assert err <= tol * float(np.abs(F).max())
+    np.testing.assert_array_equal(c.get(6), c.get3(6).T)
+    d = stages({"lang_on": 0}, m, prec)
+    d.restore(c.checkpoint())
+    np.testing.assert_array_equal(d.get(6), c.get(6))
+    c.close()
+    d.close()
+    large = M.replicate(protein(41, 34), 100, 300.0 * A, 34)
+    b = G.Batch(p, [large, m], seeds=[3, 3], precision=prec)
+    b.run(1)
+    err = float(np.abs(b.get(1, 6) - F).max())
+    assert err <= tol * float(np.abs(F).max())
+    b.close()
+
+
 def test_forces_outside_a_step_are_the_arrays_forces():
     # mixed precision accumulates in FP64: what an evaluation leaves, what a
     # reader gets and what an integration takes are the same FP32 forces
