@@ -830,20 +830,27 @@ __device__ __forceinline__ uint32_t add4(uint32_t x, uint32_t y) {
 __device__ __forceinline__ uint32_t sub4(uint32_t x, uint32_t y) {
   return ((x | 0x80808080u) - (y & 0x7f7f7f7fu)) ^ ((x ^ ~y) & 0x80808080u);
 }
-// LDS of the QA finish beside the budgets: the candidates and the removed
-// contacts, as they come and in the order they are taken
+// LDS of the QA finish beside the budgets: the candidates as they come and in
+// the order they are taken, and the removed contacts as they come
 struct QfLds {
   long long key[QF_CAND_LDS];   // by distance; then the accepted ones' ranks
   uint64_t sd[QF_CAND_LDS];     // by rank: budget changes of the two residues,
   int i1[QF_CAND_LDS], i2[QF_CAND_LDS], sc[QF_CAND_LDS];  // the residues, the slot
   int idx[QF_CAND_LDS];
-  uint64_t rsd[QF_REM_LDS];     // by rank
-  int ri1[QF_REM_LDS], ri2[QF_REM_LDS];
-  int rem[QF_REM_LDS];          // as they come: 2 * contact + near
+  int rem[QF_REM_LDS];          // 2 * contact + near
   int wave[16];
   int near, accepted, live, overflow;
 };
 
+// budget word w takes the four changes in d (they commute: any order)
+__device__ __forceinline__ void give_back(uint32_t *w, uint32_t d) {
+  uint32_t old = *w;
+  for (;;) {
+    const uint32_t seen = atomicCAS(w, old, add4(old, d));
+    if (seen == old) return;
+    old = seen;
+  }
+}
 // qa_finish_block (pcg_stages.hpp) by a whole workgroup of 1024, the budgets
 // in LDS (sy: one word of four a residue). Removed contacts and candidates are
 // ranked in parallel, one thread decides which candidates are taken, in order,
@@ -851,6 +858,7 @@ struct QfLds {
 // that thread writing the lists too, a contact cost some 1 us of waits on HBM:
 // 18 us a step for the box of 6400 residues and 1240 us for its first, where
 // it is 8 and 316 so; what is left is the chain of loads and barriers.)
+// Removed contacts beyond QF_REM_LDS are ranked where they are, in HBM.
 __device__ __forceinline__ void qa_finish_wide(const DevBatch &b, SysDescC &sd, SysState &st,
                                                uint32_t *sy, QfLds &q, int cand_n, int rem_n) {
   const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wv = tid >> 6;
@@ -861,9 +869,11 @@ __device__ __forceinline__ void qa_finish_wide(const DevBatch &b, SysDescC &sd, 
     q.key[c] = total_key(b.cand_dist[sd.nl0 + c]);
     q.idx[c] = b.cand_idx[sd.nl0 + c];
   }
+  const bool rem_lds = rem_n <= QF_REM_LDS;
   for (int a = tid; a < rem_n; a += nt) {
-    const int v = b.rem[sd.qc0 + a];
-    q.rem[a] = 2 * v + (b.qc_d[sd.qc0 + v] > b.P->qa_max_req ? 0 : 1);
+    const int v = b.rem[sd.qc0 + a], w = 2 * v + (b.qc_d[sd.qc0 + v] > b.P->qa_max_req ? 0 : 1);
+    if (rem_lds) q.rem[a] = w;
+    else b.rem[sd.qc0 + a] = w;
   }
   for (int k = tid; k < sd.n; k += nt) sy[k] = *(const uint32_t *)(b.sync + 4 * (r0 + k));
   __syncthreads();
@@ -883,19 +893,26 @@ __device__ __forceinline__ void qa_finish_wide(const DevBatch &b, SysDescC &sd, 
     q.sd[rank] = *(const uint64_t *)(b.cand_sd + 8 * (size_t)sc);
   }
   // removed contacts in increasing index order, back among the free pairs
+  const int *rem_hbm = b.rem + sd.qc0;
   for (int a = tid; a < rem_n; a += nt) {
-    const int v = q.rem[a] >> 1, near = q.rem[a] & 1, qc = sd.qc0 + v;
+    const int own = rem_lds ? q.rem[a] : rem_hbm[a];
+    const int v = own >> 1, near = own & 1, qc = sd.qc0 + v;
     int rank = 0, nearer = 0;
-    for (int o = 0; o < rem_n; ++o) {
-      const int w = q.rem[o];
+    auto behind = [&](int o, int w) {
       const bool before = (w >> 1) < v || ((w >> 1) == v && o < a);
       rank += before ? 1 : 0;
       nearer += before ? (w & 1) : 0;
+    };
+    if (rem_lds) {
+      for (int o = 0; o < rem_n; ++o) behind(o, q.rem[o]);
+    } else {
+#pragma clang loop unroll_count(8)
+      for (int o = 0; o < rem_n; ++o) behind(o, rem_hbm[o]);
     }
     const int i1 = b.qc_i[0][qc], i2 = b.qc_i[1][qc];
-    q.ri1[rank] = i1 - r0;
-    q.ri2[rank] = i2 - r0;
-    q.rsd[rank] = *(const uint64_t *)(b.qc_sd + 8 * (size_t)qc);
+    const uint64_t back = *(const uint64_t *)(b.qc_sd + 8 * (size_t)qc);
+    give_back(sy + (i1 - r0), (uint32_t)back);
+    give_back(sy + (i2 - r0), (uint32_t)(back >> 32));
     b.qc_vac[qc] = 1;
     const int slot = store0 + rank;
     if (slot >= sd.qfcap) {
@@ -922,11 +939,6 @@ __device__ __forceinline__ void qa_finish_wide(const DevBatch &b, SysDescC &sd, 
   __syncthreads();
   int *taken = (int *)q.key;
   if (tid == 0) {
-    for (int a = 0; a < rem_n; ++a) {
-      const uint64_t v = q.rsd[a];
-      sy[q.ri1[a]] = add4(sy[q.ri1[a]], (uint32_t)v);
-      sy[q.ri2[a]] = add4(sy[q.ri2[a]], (uint32_t)(v >> 32));
-    }
     int n = 0;
     for (int a = 0; a < cand_n; ++a) {
       const int i1 = q.i1[a] - r0, i2 = q.i2[a] - r0;
@@ -1016,8 +1028,8 @@ __device__ __forceinline__ void qa_finish_wide(const DevBatch &b, SysDescC &sd, 
 }
 
 // The QA finish of a step, one workgroup a system: qa_finish_wide where the
-// budgets fit its LDS (sync_lds) and the candidates and removals their
-// staging, which only the first steps of a large system outgrow.
+// budgets fit its LDS (sync_lds) and the candidates their staging, which only
+// the first steps of a large system outgrow.
 __global__ __launch_bounds__(1024) void k_qa_finish(DevBatch b, int sync_lds) {
   extern __shared__ __align__(16) unsigned char qf_lds[];
   int s = blockIdx.x;
@@ -1034,7 +1046,7 @@ __global__ __launch_bounds__(1024) void k_qa_finish(DevBatch b, int sync_lds) {
   const int n = sd.n, r0 = sd.res0;
   QfLds &q = *(QfLds *)qf_lds;
   uint32_t *syl = (uint32_t *)(qf_lds + sizeof(QfLds));
-  if (cand_n <= QF_CAND_LDS && rem_n <= QF_REM_LDS) {
+  if (cand_n <= QF_CAND_LDS) {
     qa_finish_wide(b, sd, st, syl, q, cand_n, rem_n);
     return;
   }

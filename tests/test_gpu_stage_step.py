@@ -163,3 +163,36 @@ def test_qa_contacts_form_break_and_are_compressed(copies, side, steps):
     np.testing.assert_array_equal(np.stack(ours[:2]), np.stack(ref[:2]))
     assert np.abs(c.get(0) - o.r()).max() < 1e-8
     c.close()
+
+
+@pytest.mark.parametrize("copies,side", [(20, 70.0), (60, 110.0)])
+def test_most_qa_contacts_break_in_one_step(copies, side):
+    # the positions grow by a factor of two: nearly all contacts break at once,
+    # in the first case just as many as the finish keeps in its LDS, in the
+    # second more; and form again at half the size
+    over = {"qa_phase_dur": 0.02, "nat_cont_on": 0, "temperature": 3.0}
+    m = M.replicate(protein(41, 34), copies, side * A, 34)
+    o, c = Oracle(dict(FULL, **over), m, seed=3), stages(over, m)
+    o.set_noise_scale(0.0)
+    o.step(4)
+    c.step(4)
+    for grow in (2.0, 0.5, 1.0):
+        r = o.r() * grow
+        o.set_r(r)
+        c.set(0, r)
+        o.fix_nl()  # (a context's step looks at what its own steps moved)
+        c.fix_nl()
+        before = o.num_qa_contacts()
+        o.step(1)
+        c.step(1)
+        sync, num = c.qa_state()
+        assert num == o.num_qa_contacts()
+        np.testing.assert_array_equal(sync, o.sync())
+        ours, ref = c.list(6), o.list(6)
+        np.testing.assert_array_equal(np.stack(ours[:2]), np.stack(ref[:2]))
+        ours, ref = c.list(5), o.list(5)
+        np.testing.assert_array_equal(np.stack(ours[:2]), np.stack(ref[:2]))
+        np.testing.assert_array_equal(ours[3] != 0, ref[3] != 0)
+        if grow > 1.0:
+            assert (before > 512) == (copies == 60)
+    c.close()
