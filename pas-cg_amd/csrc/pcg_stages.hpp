@@ -131,8 +131,12 @@ __device__ inline void qa_finish_block(const DevBatch &b, SysDescC &sd, SysState
     for (int o = 0; o < cand_n; ++o) {
       int so = sd.nl0 + o;
       long long kd = total_key(b.cand_dist[so]);
-      const int io = b.cand_idx[so];
-      rank += (kd < kc || (kd == kc && (io < ic || (io == ic && o < c)))) ? 1 : 0;
+      if (kd == kc) {  // (the rare case loads the second key)
+        const int io = b.cand_idx[so];
+        rank += (io < ic || (io == ic && o < c)) ? 1 : 0;
+      } else {
+        rank += kd < kc ? 1 : 0;
+      }
     }
     b.cand_perm[sd.nl0 + rank] = c;
   }
