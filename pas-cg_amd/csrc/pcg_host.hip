@@ -1440,6 +1440,11 @@ void enqueue_step(DeviceBatch &B, const double *noise = nullptr) {
   if (B.hp.ljw_terms) launch_ljw_process(d, B.stream);
   launch_lang(d, B.prec, B.noise, noise, B.stream, true, B.box_set);
 }
+// how many launches that is
+int step_launches(const DeviceBatch &B) {
+  return (B.box_set ? 1 : 0) + fix_nl_launches(B.max_n, B.cell_words) + 1 + (B.hp.p.qa_on ? 1 : 0) +
+         (B.hp.ljw_terms ? 1 : 0) + 1;
+}
 
 // the host copy of the system descriptor after the box protocol moved the
 // PBC cell on the device
@@ -2097,7 +2102,7 @@ int run_stages(pcg_batch *b, int nsteps) {
   float ms = 0.f;
   HIPCHK(hipEventElapsedTime(&ms, b->ev0, b->ev1));
   b->last_ms = ms;
-  b->last_launches = nsteps * 8;
+  b->last_launches = nsteps * step_launches(B);
   return PCG_OK;
 }
 

@@ -1576,6 +1576,9 @@ void launch_fix_nl(const DevBatch &b, int max_n, int cell_words, hipStream_t s, 
   hipLaunchKernelGGL(k_nl_rows<true>, rg, dim3(BLK), mask_lds, s, b, cell_words, fuse, 0, 0);
   if (!step) hipLaunchKernelGGL(k_nl_done, dim3((unsigned)b.nsys), dim3(BLK), 0, s, b);
 }
+int fix_nl_launches(int max_n, int cell_words) {
+  return (cell_words > 0 ? 2 : 0) + (max_n < ROWS_FUSE_MAX ? 2 : 3);
+}
 void launch_terms(const DevBatch &b, int prec, int max_items, int term, int from, int to,
                   hipStream_t s) {
   int gx = (max_items + BLK - 1) / BLK;

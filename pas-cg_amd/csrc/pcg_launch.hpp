@@ -40,6 +40,8 @@ void launch_prepare_nh(const DevBatch &b, hipStream_t s);
 // the rebuild is closed here.
 void launch_fix_nl(const DevBatch &b, int max_n, int cell_words, hipStream_t s, bool step,
                    int qa_on);
+// and its launches in a step
+int fix_nl_launches(int max_n, int cell_words);
 // every term, of a step or (step false) of an evaluation outside one
 void launch_step_terms(const DevBatch &b, int prec, int max_n, bool step, hipStream_t s);
 // a single term outside a step

@@ -129,6 +129,16 @@ def test_forces_of_steps_without_langevin(prec, tol):
     b.close()
 
 
+@pytest.mark.parametrize("qa_on", [1, 0])
+def test_launches_of_a_batch_on_the_stage_kernels(qa_on):
+    # cells (two), rows, their scan, rows, terms, QA finish, Langevin
+    large = M.replicate(protein(41, 34), 100, 300.0 * A, 34)
+    b = G.Batch(dict(FULL, qa_on=qa_on), [large], precision=G.MIXED)
+    b.run(3)
+    assert b.last_ms()[1] == 3 * (7 + qa_on)
+    b.close()
+
+
 def test_forces_outside_a_step_are_the_arrays_forces():
     # mixed precision accumulates in FP64: what an evaluation leaves, what a
     # reader gets and what an integration takes are the same FP32 forces
