@@ -303,8 +303,9 @@ int pcg_use_graph(pcg_ctx *c, int32_t on);
  * system (one workgroup, many steps a launch, positions, forces and lists
  * in LDS), possible when the system fits LDS, the noise is Philox and there
  * are no walls or box (PCG_E_STATE otherwise). PCG_FORM_AUTO (the default)
- * takes the persistent form whenever it is possible and the faster one:
- * below 700 residues with QA, below 900 without. The first step in one
+ * takes the persistent form whenever it is possible and the system is small
+ * (below 700 residues with QA, 900 without, about where the stages become
+ * the faster form in either precision). The first step in one
  * form after steps in the other rebuilds the neighbour list, and so does the
  * first nl_verify after persistent steps; per-term calls right after
  * persistent steps see the lists of the persistent kernel's last rebuild,

@@ -361,7 +361,6 @@ struct Arena {
 
 } // namespace
 
-// A device batch: the systems, their arena and the launch configuration.
 // Pinned host memory that kernels write results into, grown as asked for and
 // kept for the next result of its owner; behind it, the sequence number of the
 // last fetch that has arrived and the overflow flag of the step kernels.
@@ -389,6 +388,7 @@ struct Pinned {
   }
 };
 
+// A device batch: the systems, their arena and the launch configuration.
 struct DeviceBatch {
   int prec = PCG_MIXED;
   int noise = PCG_NOISE_PHILOX;
@@ -1461,10 +1461,16 @@ bool persistent_eligible(const pcg_ctx &c) {
   return c.pcfg.ok && B.noise == PCG_NOISE_PHILOX && B.hp.p.n_walls == 0 && !B.box_set;
 }
 // PCG_FORM_AUTO: one workgroup's step grows with the system, the stages' is
-// their launches. us a step, persistent and stages, mixed precision: without
-// QA 500 residues 14 and 24, 700 18 and 24, 800 23 and 24, 900 26 and 24,
-// 1200 37 and 27; with QA 500 24 and 28, 600 31 and 29, 700 29 and 27, 900 42
-// and 28, 2000 148 and 36. The stages' forces are no less precise: they
+// their launches. us a step, persistent and stages, mixed precision | FP64:
+//   no QA  500 residues 14, 25 | 15, 25; 700 18, 24 | 19, 25; 850 24, 24 | 26, 25;
+//          900 26, 25 | 28, 25; 1200 37, 27 | 39, 28
+//   QA     500 23, 28 | 24, 29; 650 27, 27 | 29, 27; 700 29, 28 | 30, 28;
+//          800 35, 28 | 37, 29; 1200 58, 31 | 60, 31; 2000 148, 36 (mixed)
+//   no QA, Pauli and DH: 700 22, 25 | 24, 26; 750 26, 25 | 27, 26; 900 35, 26 | 36, 26
+// The forms cross between 600 and 700 residues with QA and between 700 and 850
+// without, a little earlier in FP64 and with the density of the protein (a
+// compact one of 600 with QA takes 31, 30 | 33, 30); the lines are where the
+// stages win in both precisions. The stages' forces are no less precise: they
 // accumulate in FP64 and take the bonded terms in FP64.
 bool use_persistent(const pcg_ctx &c) {
   if (c.form != PCG_FORM_AUTO) return c.form == PCG_FORM_PERSISTENT;

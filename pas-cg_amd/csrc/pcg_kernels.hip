@@ -1091,7 +1091,7 @@ __device__ __forceinline__ void box_log(const DevBatch &b) {
 
 // time and energy bookkeeping at the end of a step (step.cpp:157-162)
 // v: the sum of its energies
-__device__ __forceinline__ void tick_system(const DevBatch &b, int s, int advance, int nl_done,
+__device__ __forceinline__ void tick_system(const DevBatch &b, int s, int advance, bool nl_done,
                                             double v) {
   SysState &st = b.st[s];
   // (all reads first: one wait instead of one for each)
@@ -1118,11 +1118,12 @@ __device__ __forceinline__ double sum_energies(const SysState &st) {
   return v;
 }
 
-__global__ void k_tick(DevBatch b, int advance, int nl_done) {
+// the tick outside a step, where k_nl_done closes rebuilds
+__global__ void k_tick(DevBatch b, int advance) {
   int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= b.nsys) return;
   if (!b.st[s].active) return;
-  tick_system(b, s, advance, nl_done, sum_energies(b.st[s]));
+  tick_system(b, s, advance, false, sum_energies(b.st[s]));
 }
 
 
@@ -1196,7 +1197,7 @@ __global__ void k_lang(DevBatch b, int noise_mode, const double *noise, int tick
     if (__any(done >= 0))
       for (int k = 0; k < NT; ++k) v += __shfl(vk, k, 64);
     if (done >= 0) {
-      tick_system(b, done, 1, 1, done == sys0 ? v : sum_energies(b.st[done]));
+      tick_system(b, done, 1, true, done == sys0 ? v : sum_energies(b.st[done]));
       b.st[done].done_lang = 0;
     }
   }
@@ -1605,7 +1606,7 @@ size_t qa_finish_lds(int max_n) {
   return sizeof(QfLds) + 4 * (((size_t)max_n + 1) & ~(size_t)1);
 }
 void launch_qa_finish(const DevBatch &b, int max_n, hipStream_t s) {
-  // the budgets in LDS while they and the candidates fit 96 KB
+  // the budgets in LDS while they and the candidates fit QF_LDS_MAX
   const size_t lds = qa_finish_lds(max_n);
   const int sync_lds = lds <= QF_LDS_MAX ? max_n : 0;
   hipLaunchKernelGGL(k_qa_finish, dim3(b.nsys), dim3(1024), sync_lds ? lds : 0, s, b, sync_lds);
@@ -1620,8 +1621,8 @@ void launch_lang(const DevBatch &b, int prec, int noise_mode, const double *nois
   else
     hipLaunchKernelGGL(k_lang<float>, g, dim3(BLK), 0, s, b, noise_mode, noise, t, l);
 }
-void launch_tick(const DevBatch &b, int advance, hipStream_t s, bool nl_done) {
-  hipLaunchKernelGGL(k_tick, grid1(b.nsys, 64), dim3(64), 0, s, b, advance, nl_done ? 1 : 0);
+void launch_tick(const DevBatch &b, int advance, hipStream_t s) {
+  hipLaunchKernelGGL(k_tick, grid1(b.nsys, 64), dim3(64), 0, s, b, advance);
 }
 void launch_ljw_process(const DevBatch &b, hipStream_t s) {
   hipLaunchKernelGGL(k_ljw_process, dim3(1), dim3(1024), 0, s, b);

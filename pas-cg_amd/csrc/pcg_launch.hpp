@@ -53,7 +53,7 @@ void launch_qa_finish(const DevBatch &b, int max_n, hipStream_t s);
 // noise: RAN2 draws in host memory, or null for those on the device
 void launch_lang(const DevBatch &b, int prec, int noise_mode, const double *noise, hipStream_t s,
                  bool tick = false, bool log = false);
-void launch_tick(const DevBatch &b, int advance, hipStream_t s, bool nl_done = false);
+void launch_tick(const DevBatch &b, int advance, hipStream_t s);
 // walls and the box protocol of a plain context (b.wall set): LJ candidate
 // processing; box set-up, and the phase logic before a step. P and sd are the
 // writable device parameters and system descriptor.

@@ -1037,8 +1037,8 @@ __device__ __forceinline__ bool nl_moved(DevBatchC *bp, int s, const SysState &s
 // or not chain-local, the simple native dihedral, disulfide contacts, PID
 // pairs, the relative Debye-Hueckel term and walls. A step is a chain of
 // short dependent phases, bound by latency and instruction issue, and the
-// general form's unused code was most of the kernel: 25 000 instructions
-// against 12 000, 179 spilled VGPRs against 56 on 1024 threads. With LEAN,
+// general form's unused code is half of the kernel: 23 600 instructions
+// against 12 400, 204 spilled VGPRs against 65 on 1024 threads. With LEAN,
 // unpack() and the step's decisions taken by every thread, a step of one
 // 56-residue Go chain takes 5.5 us instead of 9.4, of a 301-residue protein
 // in the full force field 17.3 us instead of 22.0.
