@@ -746,10 +746,10 @@ template <int T> struct Term {
 // device, so the grid follows the work. A wave's chunk is a serial chain of
 // some thousand instructions on almost empty SIMDs, which bounds the kernel: a
 // grid of blocks for every term at its largest size was 11 000 blocks, nearly
-// all empty, and took 17.4 us for a box of 6400 residues, 18 for 2000 in one
-// chain and 13.1 for 480 between walls; this one takes 13.2, 15.7 and 11.1
-// (29 and more with one chunk of all the bonded items). Also resets what the
-// step's verify read.
+// all empty, and took 18.4 us for a box of 64 chains of 100, 18 for 2000
+// residues in one chain and 12.9 for 480 between walls; this one takes 14.0,
+// 15.5 and 10.3 (29 and more with one chunk of all the bonded items). Also
+// resets what the step's verify read.
 template <typename R> __global__ __launch_bounds__(BLK) void k_step_terms(DevBatch b, int step) {
   const int s = blockIdx.y;
   SysState &st = b.st[s];
@@ -856,8 +856,8 @@ __device__ __forceinline__ void give_back(uint32_t *w, uint32_t d) {
 // ranked in parallel, one thread decides which candidates are taken, in order,
 // on LDS alone, and the lists are written and compressed in parallel. (With
 // that thread writing the lists too, a contact cost some 1 us of waits on HBM:
-// 18 us a step for the box of 6400 residues and 1240 us for its first, where
-// it is 8 and 316 so; what is left is the chain of loads and barriers.)
+// 11 us a step for a box of 64 chains of 100 and 2400 us for its first, where
+// it is 6.7 and 575 so; what is left is the chain of loads and barriers.)
 // Removed contacts beyond QF_REM_LDS are ranked where they are, in HBM.
 __device__ __forceinline__ void qa_finish_wide(const DevBatch &b, SysDescC &sd, SysState &st,
                                                uint32_t *sy, QfLds &q, int cand_n, int rem_n) {
